@@ -649,13 +649,27 @@ static dim3 gemm_grid(uint32_t rows, uint32_t ntok, uint32_t nz, uint32_t rows_p
     return dim3((rows + rows_per_wg - 1) / rows_per_wg, (ntok + tokens_per_wg - 1) / tokens_per_wg, nz);
 }
 
+// Calls of up to SMALL_TOKENS tokens run the small-call kernels (token-blocked
+// activations, 32-token tiles, split K): a 4-layer block of the model (one layer of
+// each kind) at 129 / 203 / 512 / 700 tokens takes 0.70 / 0.76 / 1.09 / 1.38 ms against
+// 1.23 / 1.24 / 1.26 / 1.43 ms with the large-call kernels, whose 128-token tiles leave
+// most CUs idle (a 2048-row projection of 203 tokens is 32 workgroups) and most of an
+// expert's tile empty; with whole-range int8 scales 0.68 / 0.83 / 1.32 / 1.64 ms against
+// 1.44 / 1.48 / 1.75 / 1.99.  At 1024 tokens the two meet (1.72 against 1.67 ms).
+#define SMALL_TOKENS 704u
+// (models narrower than two Q6_K blocks keep to GEMM_TOKENS: their projections
+// cannot be split over K, so no reduce would leave the router partial sums that
+// the expert lists of more than 256 tokens are formed from)
+static bool small_call(uint32_t T, uint32_t dim) { return T <= (dim >= 512 ? SMALL_TOKENS : (uint32_t)GEMM_TOKENS); }
+
 #define GEMM_PART_BYTES ((size_t)64 << 20) // split-K partial sums (prefill scratch)
 #define GEMM_PART_SOFT ((size_t)1600000) // small calls' partial sums, floats (6.4 MB)
 #define GEMM_N64_BELOW 512u // two 128-token workgroups per CU on 256 CUs
 
 // Launches the matrix-core GEMM g (pair: gate + up + SwiGLU) over T tokens and nz
-// groups.  Up to one 128-token tile (T <= 128, as in 64-token chunked prefill,
-// about 8 tokens per expert) the kernels with 32-token tiles run, the grid is
+// groups.  Small calls (`small`: activations in the token-blocked layout, e.g. the
+// 64-token chunks of a prefill, about 8 tokens per expert) run the kernels with
+// 32-token tiles; the grid is
 // then mostly the weight-row tiles and each workgroup's K loop is a chain of
 // dependent stages, so K is split into slices (about 1024 workgroups, each slice
 // at least one Q6_K block, the partials within `part_cap` floats of `part` and
@@ -674,7 +688,7 @@ struct RouterPart {
     uint32_t *counts; // nullable: zeroed by the reduce (the next split counts into it)
 };
 
-static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, uint32_t T, uint32_t nz,
+static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool small, uint32_t T, uint32_t nz,
                        uint32_t part_rows, uint32_t n_used, float *part, size_t part_cap, uint64_t *dispatches,
                        const CombinePrefillArgs *combine = nullptr, bool *combined = nullptr,
                        uint32_t *deferred = nullptr, const RouterPart *router = nullptr, bool *router_done = nullptr,
@@ -684,7 +698,6 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, uint32_
         *router_done = false;
     if (combined)
         *combined = false;
-    const bool small = T <= GEMM_TOKENS;
     // weights with scales outside [-64, 64] take the split-scale kernels (one 32-row
     // tile per wave for small single-weight calls, 64 tokens per large workgroup)
     const bool exact = g.w.wide || (pair && g.w2.wide);
@@ -710,6 +723,8 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, uint32_
         // adding them costs more than the wider grid gains (the 6144-row in_proj at
         // four slices, the dense gate/up pair unsplit, the dense down at twelve)
         S = (uint32_t)std::max<size_t>(1, std::min<size_t>(S, std::min<size_t>(part_cap, GEMM_PART_SOFT) / per));
+        if (router && g.w.nb > 1) // the reduce leaves the router partial sums
+            S = std::max(S, 2u);
         if (g.y_hi) // the split output is formed in the epilogue from whole sums
             S = 1;
     }
@@ -828,7 +843,7 @@ extern "C" int lfm_q6k_gemm(const void *packed, uint64_t rows, uint64_t in_dim, 
     }
     uint64_t nd = 0;
     if (rc == LFM_OK)
-        rc = launch_gemm(K, s, ga, false, T, 1, T, 0, part, part_cap, &nd);
+        rc = launch_gemm(K, s, ga, false, T <= GEMM_TOKENS, T, 1, T, 0, part, part_cap, &nd);
     if (rc == LFM_OK && hipStreamSynchronize(s) != hipSuccess)
         rc = fail(LFM_EDEVICE, "lfm_q6k_gemm: synchronize failed");
     (void)hipFree(hi);
@@ -1706,7 +1721,7 @@ extern "C" int lfm_engine_finalize(lfm_engine *e)
         const size_t wide = std::max<size_t>((size_t)hp.n_ff, 4 * (size_t)hp.expert_ff);
         // row-major hi / lo of a large call, or the token-blocked ones of a small call
         // (rows padded to 32; the grouped expert inputs reserve a padded list per expert)
-        const size_t ts = (std::min<size_t>(TC, GEMM_TOKENS) + 31) / 32 * 32;
+        const size_t ts = (std::min<size_t>(TC, SMALL_TOKENS) + 31) / 32 * 32;
         const size_t kmax = std::max<size_t>({(size_t)dim, (size_t)hp.n_ff, (size_t)hp.expert_ff});
         const size_t hmax = std::max<size_t>({TC * dim, TC * hp.n_ff, TC * 4 * hp.expert_ff, ts * kmax,
                                               E * ts * std::max<size_t>(dim, hp.expert_ff)});
@@ -1732,7 +1747,7 @@ extern "C" int lfm_engine_finalize(lfm_engine *e)
             HIPCHK(hipMalloc(&e->pf.lo2, h2 * 2));
         }
         HIPCHK(hipMalloc(&e->pf.cstate, (size_t)dim * 2 * 4));
-        const size_t tsmall = std::min<size_t>(TC, GEMM_TOKENS);
+        const size_t tsmall = std::min<size_t>(TC, SMALL_TOKENS);
         HIPCHK(hipMalloc(&e->pf.rpart, tsmall * (dim / 256) * E * 4));
         HIPCHK(hipMalloc(&e->pf.rss, tsmall * (dim / 256) * 4));
         HIPCHK(hipMalloc(&e->pf.logits, TC * E * 4));
@@ -1822,7 +1837,7 @@ extern "C" void lfm_engine_destroy(lfm_engine *e)
 // residual in row T - 1 of pf.x, which the head reads.
 // RMSNorm (optional) + binary16 hi / lo split of `rows` activation rows for a
 // GEMM of a T-token call: row-major for large calls, token-blocked for the
-// small-call kernels (T <= GEMM_TOKENS), whose B reads expect that layout.
+// small-call kernels (small_call), whose B reads expect that layout.
 // grouped: the rows feed the expert GEMMs; spr = expert slots per row (4 for
 // the token rows of the gate/up input, 1 for the slot rows of the down input).
 // The split's arguments for `rows` rows of width K in a call of T tokens.
@@ -1840,7 +1855,7 @@ static SplitArgs split_args(lfm_engine *e, const float *x, const float *norm, ui
     a.bscale = e->pf.bscale;
     a.T = rows;
     a.K = K;
-    a.mode = T > GEMM_TOKENS ? SPLIT_ROWMAJOR : grouped ? SPLIT_GROUPED : SPLIT_BLOCKED;
+    a.mode = !small_call(T, e->hp.dim) ? SPLIT_ROWMAJOR : grouped ? SPLIT_GROUPED : SPLIT_BLOCKED;
     if (a.mode == SPLIT_GROUPED) {
         a.sel = e->pf.sel;
         a.pos = e->pf.pos;
@@ -1922,7 +1937,7 @@ static int pf_gemm(lfm_engine *e, const Q6Tiles &w, uint32_t T, float *c, uint32
     g.ldc = ldc;
     g.col0 = col0;
     g.mode = mode;
-    return launch_gemm(e->K, e->stream, g, false, T, 1, T, 0, e->pf.part, GEMM_PART_BYTES / 4, &e->dispatches,
+    return launch_gemm(e->K, e->stream, g, false, small_call(T, e->hp.dim), T, 1, T, 0, e->pf.part, GEMM_PART_BYTES / 4, &e->dispatches,
                        nullptr, nullptr, deferred, router, router_done);
 }
 
@@ -1946,7 +1961,8 @@ static int pf_gemm_swiglu(lfm_engine *e, const Q6Tiles &wg, const Q6Tiles &wu, u
     g.zrows = zrows;
     g.c = c;
     g.ldc = ldc;
-    if (T <= GEMM_TOKENS) {
+    const bool small = small_call(T, e->hp.dim);
+    if (small) {
         if (zrows % 128)
             return fail(LFM_EINTERNAL, "prefill: split SwiGLU output needs rows in 128s, not %u", zrows);
         g.y_hi = e->pf.hi2;
@@ -1954,13 +1970,13 @@ static int pf_gemm_swiglu(lfm_engine *e, const Q6Tiles &wg, const Q6Tiles &wu, u
         g.y_bscale = e->pf.bscale2;
     }
     if (!tok)
-        return launch_gemm(e->K, e->stream, g, true, T, 1, T, 0, e->pf.part, GEMM_PART_BYTES / 4, &e->dispatches);
+        return launch_gemm(e->K, e->stream, g, true, small, T, 1, T, 0, e->pf.part, GEMM_PART_BYTES / 4, &e->dispatches);
     g.tok = tok;
     g.slot = e->pf.slot;
     g.counts = e->pf.counts;
     g.list_stride = e->ctx;
     g.rpz = (T + 31) / 32 * 32;
-    return launch_gemm(e->K, e->stream, g, true, T, e->hp.n_expert, 4 * T, e->hp.n_used, e->pf.part,
+    return launch_gemm(e->K, e->stream, g, true, small, T, e->hp.n_expert, 4 * T, e->hp.n_used, e->pf.part,
                        GEMM_PART_BYTES / 4, &e->dispatches);
 }
 
@@ -1986,7 +2002,7 @@ static int pf_gemm_grouped(lfm_engine *e, const Q6Tiles &w, uint32_t zrows, uint
     g.zrows = zrows;
     g.c = c;
     g.ldc = ldc;
-    return launch_gemm(e->K, e->stream, g, false, T, e->hp.n_expert, 4 * T, e->hp.n_used, e->pf.part,
+    return launch_gemm(e->K, e->stream, g, false, small_call(T, e->hp.dim), T, e->hp.n_expert, 4 * T, e->hp.n_used, e->pf.part,
                        GEMM_PART_BYTES / 4, &e->dispatches, combine, combined, nullptr, nullptr, nullptr,
                        defer_combine);
 }
@@ -1997,7 +2013,7 @@ static int pf_out_proj(lfm_engine *e, uint32_t l, const Q6Tiles &w, uint32_t T)
 {
     const lfm_hparams &hp = e->hp;
     e->pf.router_ready = false;
-    if (l >= hp.dense_lead && T <= GEMM_TOKENS) {
+    if (l >= hp.dense_lead && small_call(T, hp.dim)) {
         const RouterPart rp{f32(e, "blk.%u.ffn_norm.weight", l), f32(e, "blk.%u.ffn_gate_inp.weight", l), e->pf.rpart,
                             e->pf.rss, hp.n_expert, e->pf.counts};
         return pf_gemm(e, w, T, e->pf.x, hp.dim, 0, 1, nullptr, &rp, &e->pf.router_ready);
@@ -2009,6 +2025,7 @@ static int pf_mixer(lfm_engine *e, uint32_t l, uint32_t T, uint32_t start)
 {
     const lfm_hparams &hp = e->hp;
     const uint32_t dim = hp.dim, kv = hp.kv_heads[l];
+    const bool small = small_call(T, dim);
     RC(pf_split(e, e->pf.x, f32(e, "blk.%u.attn_norm.weight", l), T, dim, T));
     if (kv == 0) {
         // in_proj; with a K split the conv adds the slices itself (no reduce launch)
@@ -2016,7 +2033,7 @@ static int pf_mixer(lfm_engine *e, uint32_t l, uint32_t T, uint32_t start)
         RC(pf_gemm(e, q6tiles(e, "blk.%u.shortconv.in_proj.weight", l), T, e->pf.bcx, 3 * dim, 0, 0, &S));
         ConvPrefillArgs c{S > 1 ? e->pf.part : e->pf.bcx, f32(e, "blk.%u.shortconv.conv.weight", l), e->conv[l],
                           e->pf.cstate, e->pf.y, T, dim, S, nullptr, nullptr, nullptr};
-        if (T <= GEMM_TOKENS) { // small calls: the conv stores y split for the out projection
+        if (small) { // small calls: the conv stores y split for the out projection
             if (dim % 256)
                 return fail(LFM_EINTERNAL, "prefill conv: width %u not a multiple of 256", dim);
             c.y_hi = e->pf.hi;
@@ -2024,7 +2041,7 @@ static int pf_mixer(lfm_engine *e, uint32_t l, uint32_t T, uint32_t start)
             c.y_bscale = e->pf.bscale;
         }
         RC(launch(e->K->conv_prefill, dim3((dim + 255) / 256, T), 0, e->stream, c));
-        if (T <= GEMM_TOKENS) // the FFN's split moves the new conv state into place
+        if (small) // the FFN's split moves the new conv state into place
             e->pf.state_pending = e->conv[l];
         else // the split of y also moves the new conv state into place
             RC(pf_split(e, e->pf.y, nullptr, T, dim, T, false, 1, e->pf.cstate, e->conv[l], 2 * dim));
@@ -2059,7 +2076,7 @@ static int pf_mixer(lfm_engine *e, uint32_t l, uint32_t T, uint32_t start)
         RC(launch(e->K->attn_prefill, dim3(qtiles, kv, nsplit), 0, e->stream, at));
         AttnMergeSplitArgs mg{e->pf.part, e->pf.y, T, hp.heads, nsplit, nullptr, nullptr, nullptr};
         // small calls: the merge stores the output split for the output projection
-        const bool direct = T <= GEMM_TOKENS && hp.heads % 4 == 0 && hp.heads * 64 == dim;
+        const bool direct = small && hp.heads % 4 == 0 && hp.heads * 64 == dim;
         if (direct) {
             mg.y_hi = e->pf.hi;
             mg.y_lo = e->pf.lo;
@@ -2103,13 +2120,14 @@ static int pf_ffn(lfm_engine *e, uint32_t l, float *x, uint32_t T, bool defer_ok
 {
     const lfm_hparams &hp = e->hp;
     const uint32_t dim = hp.dim;
+    const bool small = small_call(T, dim);
     const float *norm = f32(e, "blk.%u.ffn_norm.weight", l);
     if (l < hp.dense_lead) {
         const uint32_t ff = hp.n_ff;
         RC(pf_split(e, x, norm, T, dim, T));
         RC(pf_gemm_swiglu(e, q6tiles(e, "blk.%u.ffn_gate.weight", l), q6tiles(e, "blk.%u.ffn_up.weight", l), ff, T,
                           nullptr, e->pf.g, ff));
-        const bool act2 = T <= GEMM_TOKENS; // small calls: the pair stored its output split
+        const bool act2 = small; // small calls: the pair stored its output split
         if (!act2)
             RC(pf_split(e, e->pf.g, nullptr, T, ff, T));
         RC(pf_gemm(e, q6tiles(e, "blk.%u.ffn_down.weight", l), T, x, dim, 0, 1, nullptr, nullptr, nullptr, act2));
@@ -2127,7 +2145,7 @@ static int pf_ffn(lfm_engine *e, uint32_t l, float *x, uint32_t T, bool defer_ok
         rg.rpart = e->pf.rpart + first * nb * E;
         rg.rss = e->pf.rss + first * nb;
         rg.nparts = (uint32_t)nb;
-    } else if (T <= GEMM_TOKENS) { // few tokens: one workgroup per (expert, token)
+    } else if (small) { // few tokens: one workgroup per (expert, token)
         RC(launch(e->K->router_small, dim3(E, T), 0, e->stream, ra));
         e->dispatches += 1;
     } else { // large calls: the FFN input's split first; the router reads its hi / lo
@@ -2144,7 +2162,6 @@ static int pf_ffn(lfm_engine *e, uint32_t l, float *x, uint32_t T, bool defer_ok
     // small calls: the split forms the expert lists itself (no k_route_group), and
     // with the out projection's router partials (and counts zeroed by its reduce) it
     // routes each token too (no k_route_topk)
-    const bool small = T <= GEMM_TOKENS;
     const bool self_route = small && e->pf.router_ready;
     if (self_route && rg.nparts > 8) // dim <= 2048 (validate_hparams): at most 8 partials
         return fail(LFM_EINTERNAL, "prefill router: %u partial sums per token > 8", rg.nparts);
