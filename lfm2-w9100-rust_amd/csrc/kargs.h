@@ -512,6 +512,21 @@ struct EmbedRowsArgs {
     uint32_t ids_inline[EMBED_INLINE_IDS];
 };
 
+// Session snapshot / restore: the floats [first, first + count) of a snapshot, whose
+// segments (in snapshot order, seg[i].at ascending) are an attention layer's K or V,
+// valid positions x kv heads x 64 floats over the binary16 cache [kv][ctx][64], or
+// (kv 0) a conv state of plain floats.  Every segment is a multiple of 64 floats.
+#define SESSION_SEGS 128 // LFM_MAX_LAYERS attention layers' K and V
+struct SessionSeg {
+    void *dev;
+    uint32_t at, kv;
+};
+struct SessionArgs {
+    float *host; // device address of pinned host memory: float `first` at host[0]
+    uint32_t first, count, nseg, ctx;
+    SessionSeg seg[SESSION_SEGS];
+};
+
 // The short-conv mixer of one layer in one launch (k_conv_mixer, k_conv_mixer_r):
 // phase A = ConvInprojArgs with one channel per wave (its gated output handed
 // on through `flow`, in.y unused); phase B = the output projection y += W g

@@ -1541,3 +1541,89 @@ extern "C" __global__ __launch_bounds__(WG_THREADS) void k_copy(const CopyArgs a
     for (uint64_t i = (uint64_t)blockIdx.x * WG_THREADS + threadIdx.x; i < a.n16; i += stride)
         a.dst[i] = a.src[i];
 }
+
+// ------------------------------------------------------------------ sessions
+// A chunk of a session snapshot written to (k_session_out) or read from
+// (k_session_in) pinned host memory by the kernel itself, converting the cache's
+// binary16 to and from the snapshot's floats on the way: 8 floats per thread, one
+// 16-byte cache access and two 16-byte host accesses, consecutive threads on
+// consecutive host addresses.  Bound by the host link; the conversion one element at
+// a time on the host, with the whole cache copied both ways, took 3.7 ms for the
+// 15.6 MB of an attention layer at 1900 positions and three conv states.
+struct SessionAt {
+    const SessionSeg *g;
+    size_t src; // half index in the cache, or float index in the conv state
+};
+__device__ __forceinline__ SessionAt session_at(const SessionArgs &a, uint32_t i)
+{
+    uint32_t lo = 0, hi = a.nseg; // the last segment with at <= i
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (a.seg[mid].at <= i)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    SessionAt r;
+    r.g = &a.seg[lo];
+    const uint32_t off = i - r.g->at, row = r.g->kv * 64;
+    if (r.g->kv) {
+        const uint32_t t = off / row, k = off - t * row;
+        r.src = ((size_t)(k >> 6) * a.ctx + t) * 64 + (k & 63);
+    } else {
+        r.src = off;
+    }
+    return r;
+}
+extern "C" __global__ __launch_bounds__(256) void k_session_out(const SessionArgs a)
+{
+    const uint32_t u = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (u >= a.count)
+        return;
+    const SessionAt w = session_at(a, a.first + u);
+    uint32_t o[8];
+    if (w.g->kv) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(reinterpret_cast<const uint16_t *>(w.g->dev) + w.src);
+        const uint32_t p[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t h = (p[j / 2] >> (16 * (j & 1))) & 0xFFFFu;
+            const uint32_t f = __builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(_Float16, (uint16_t)h));
+            // infinities and NaN keep their payload bits as they are
+            o[j] = (h & 0x7C00u) == 0x7C00u ? ((h & 0x8000u) << 16) | 0x7F800000u | ((h & 0x3FFu) << 13) : f;
+        }
+    } else {
+        const uint4 *s = reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(w.g->dev) + w.src);
+        const uint4 x = s[0], y = s[1];
+        o[0] = x.x, o[1] = x.y, o[2] = x.z, o[3] = x.w, o[4] = y.x, o[5] = y.y, o[6] = y.z, o[7] = y.w;
+    }
+    uint4 *d = reinterpret_cast<uint4 *>(a.host + u);
+    d[0] = make_uint4(o[0], o[1], o[2], o[3]);
+    d[1] = make_uint4(o[4], o[5], o[6], o[7]);
+}
+extern "C" __global__ __launch_bounds__(256) void k_session_in(const SessionArgs a)
+{
+    const uint32_t u = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (u >= a.count)
+        return;
+    const uint4 *s = reinterpret_cast<const uint4 *>(a.host + u);
+    const uint4 x = s[0], y = s[1];
+    const SessionAt w = session_at(a, a.first + u);
+    if (w.g->kv) {
+        const uint32_t f[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+        uint32_t o[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t m = f[j] & 0x7FFFFFFFu;
+            const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)__builtin_bit_cast(float, f[j])); // RNE
+            // NaN: quiet, the top payload bits kept
+            const uint32_t q = m > 0x7F800000u ? ((f[j] >> 16) & 0x8000u) | 0x7E00u | ((m >> 13) & 0x3FFu) : h;
+            o[j / 2] |= q << (16 * (j & 1));
+        }
+        *reinterpret_cast<uint4 *>(reinterpret_cast<uint16_t *>(w.g->dev) + w.src) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+        uint4 *d = reinterpret_cast<uint4 *>(reinterpret_cast<float *>(w.g->dev) + w.src);
+        d[0] = x;
+        d[1] = y;
+    }
+}

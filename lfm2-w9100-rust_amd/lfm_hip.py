@@ -238,6 +238,11 @@ def _f32p(a: np.ndarray):
     return a.ctypes.data_as(C.POINTER(C.c_float))
 
 
+# CPython's calls for a bytes object whose creator fills it in.
+_bytes_new = C.PYFUNCTYPE(C.py_object, C.c_char_p, C.c_ssize_t)(("PyBytes_FromStringAndSize", C.pythonapi))
+_bytes_at = C.PYFUNCTYPE(C.c_void_p, C.py_object)(("PyBytes_AsString", C.pythonapi))
+
+
 def device_count() -> int:
     n = C.c_int(0)
     _check(lib().lfm_device_count(C.byref(n)))
@@ -774,11 +779,15 @@ class GpuEngine:
 
     def snapshot_resident_cache(self, valid_tokens: int) -> bytes:
         n = self.snapshot_bytes(valid_tokens)
-        buf = np.empty(n, dtype=np.uint8)
+        if n == 0:
+            return b""
+        # the bytes object is made first and written in place (no other reference to
+        # it exists yet): a copy of the buffer would cost as much as the snapshot
+        out = _bytes_new(None, n)
         w = C.c_size_t(0)
         _check(lib().lfm_snapshot_cache(self._e, valid_tokens,
-                                        buf.ctypes.data_as(C.POINTER(C.c_uint8)), n, C.byref(w)))
-        return buf.tobytes()
+                                        C.cast(_bytes_at(out), C.POINTER(C.c_uint8)), n, C.byref(w)))
+        return out
 
     def restore_session(self, valid_tokens: int, data: bytes):
         a = np.frombuffer(data, dtype=np.uint8)
