@@ -702,7 +702,7 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
         *router_done = false;
     if (combined)
         *combined = false;
-    // weights with scales outside [-64, 64] take the split-scale kernels (one 32-row
+    // weights with scales outside [-64, 64] take the two-part kernels (one 32-row
     // tile per wave for small single-weight calls, 64 tokens per large workgroup)
     const bool exact = g.w.wide || (pair && g.w2.wide);
     // small ungrouped projections of up to 3072 rows (q/k/v, the out projections):

@@ -317,7 +317,7 @@ struct Q6Tiles {
     uint32_t rows;   // rows per slice (R)
     uint32_t wide;   // some sub-block scale (of a block with d != 0) lies outside
                      // [-64, 64]: its weights sc (q - 32) can exceed 2048 in
-                     // magnitude and need the GEMMs' split-scale (_x) kernels
+                     // magnitude and need the GEMMs' two-part (_x) kernels
     const uint8_t *h16; // nullable: the binary16 fragment copy below (not wide only)
 };
 

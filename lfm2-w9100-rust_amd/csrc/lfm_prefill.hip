@@ -687,46 +687,30 @@ __device__ __forceinline__ StageScales stage_scales(uint32_t sc, int q)
     return {s, s * (half2v){(_Float16)-288.0f, (_Float16)-288.0f}};
 }
 
-// The split form of the stage's scales, for weights whose products sc (q6 - 32)
-// can exceed 2048 in magnitude (a binary16 holds every integer up to 2048 only):
-// sc = sh + sl with sh = sc & ~15 (a multiple of 16) and sl = sc & 15, formed from
-// the stored byte b = sc + 128 as (b & 0xF0) - 128 and b & 15.  Both partial
-// weights are exact binary16 values for every int8 scale: sh (q6 - 32) is 16
-// times an integer of magnitude <= 256, and |sl (q6 - 32)| <= 480; so are the
-// biases -288 sh (= -9 (sh / 16) 512) and -288 sl.
-struct SplitScales {
-    half2v sh, sl;
-};
-__device__ __forceinline__ SplitScales stage_scales_split(uint32_t sc, int q)
-{
-    const uint32_t sel = q ? 0x01070006u : 0x01050004u;
-    const uint32_t vh = __builtin_amdgcn_perm(sc & 0xF0F0F0F0u, 0x64646464u, sel);
-    const uint32_t vl = __builtin_amdgcn_perm(sc & 0x0F0F0F0Fu, 0x64646464u, sel);
-    return {__builtin_bit_cast(half2v, vh) - (half2v){(_Float16)1152.0f, (_Float16)1152.0f},
-            __builtin_bit_cast(half2v, vl) - (half2v){(_Float16)1024.0f, (_Float16)1024.0f}};
-}
-
 // The 8 binary16 weights sc * (q6 - 32) of sub-block s (0..3) of a chunk, in MFMA
 // A-operand order; ss = stage_scales of the chunk for stage s / 2.  Each is one
 // fused multiply-add of the code pair's 256 + c: (256 + c) sc - 288 sc, rounded
 // once, i.e. exact while |sc * (q6 - 32)| <= 2048 and within 1/2 ulp otherwise.
 // Sub-blocks 0..2 mask their code word; sub-block 3 gathers its code's three bit
 // pairs from the other words.
+__device__ __forceinline__ uint32_t code_bits(const AChunk &c, uint32_t s, int w) // of chunk half w
+{
+    const uint32_t X0 = w ? c.ql.y : c.ql.x, X1 = w ? c.ql.w : c.ql.z, X2 = w ? c.qh.y : c.qh.x;
+    const uint32_t M1 = 0x03030303u;
+    switch (s) {
+    case 0: return X0 & ~M1;
+    case 1: return X1 & ~M1;
+    case 2: return X2 & ~M1;
+    default: return (((((X2 & M1) << 2) | (X1 & M1)) << 2) | (X0 & M1)) << 2;
+    }
+}
 __device__ __forceinline__ half8 decode_frag(const AChunk &c, uint32_t s, _Float16 scf, _Float16 bf)
 {
     const half2v sc2 = {scf, scf}, b2 = {bf, bf};
     half2v o[4];
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-        const uint32_t X0 = w ? c.ql.y : c.ql.x, X1 = w ? c.ql.w : c.ql.z, X2 = w ? c.qh.y : c.qh.x;
-        const uint32_t M1 = 0x03030303u;
-        uint32_t t;
-        switch (s) {
-        case 0: t = X0 & ~(M1); break;
-        case 1: t = X1 & ~(M1); break;
-        case 2: t = X2 & ~(M1); break;
-        default: t = (((((X2 & M1) << 2) | (X1 & M1)) << 2) | (X0 & M1)) << 2; break;
-        }
+        const uint32_t t = code_bits(c, s, w);
         o[2 * w] = __builtin_elementwise_fma(codes256(t, false), sc2, b2);
         o[2 * w + 1] = __builtin_elementwise_fma(codes256(t, true), sc2, b2);
     }
@@ -741,6 +725,33 @@ __device__ __forceinline__ half8 decode_frag(const AChunk &c, uint32_t s, const 
 __device__ __forceinline__ half8 decode_frag(const AChunk &c, uint32_t s, half2v sc)
 {
     return decode_frag(c, s, sc[s & 1], sc[s & 1] * (_Float16)-288.0f);
+}
+
+// The same weights in two exact parts, for scales outside [-64, 64], whose weights can
+// exceed 2048 in magnitude (a binary16 holds every integer up to 2048 only): w the weight
+// rounded to binary16 and r = weight - w, which is 0 or +-1 (the weights are integers of
+// magnitude at most 4096) and which one fused multiply-add forms exactly.  The GEMMs add
+// w xh, r xh and w xl; r xl is left out: |r xl| <= 2^-11 |xh| against a weight above
+// 2048, 2^-22 of the term, the precision of the activations' own split.
+struct SplitFrag {
+    half8 w, r;
+};
+__device__ __forceinline__ SplitFrag decode_frag_split(const AChunk &c, uint32_t s, _Float16 scf)
+{
+    const half2v sc2 = {scf, scf}, b2 = sc2 * (half2v){(_Float16)-288.0f, (_Float16)-288.0f};
+    half2v o[4], r[4];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const uint32_t t = code_bits(c, s, w);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const half2v q = codes256(t, h);
+            o[2 * w + h] = __builtin_elementwise_fma(q, sc2, b2);
+            r[2 * w + h] = __builtin_elementwise_fma(q - (half2v){(_Float16)288.0f, (_Float16)288.0f}, sc2, -o[2 * w + h]);
+        }
+    }
+    return {(half8){o[0][0], o[0][1], o[1][0], o[1][1], o[2][0], o[2][1], o[3][0], o[3][1]},
+            (half8){r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]}};
 }
 
 // Q6Tiles -> binary16 fragment copy (kargs.h TILE_H16): workgroup tb (one wave)
@@ -820,10 +831,12 @@ __device__ __forceinline__ void store_rows16(float *out, uint32_t rb, uint32_t z
     }
 }
 
-// EXACT: the weights are formed with the split scales (stage_scales_split), two
-// A fragments per chunk and sub-block, each multiplied by the hi and lo
-// activation halves: four matrix-core products per k-step instead of two, and
-// exact binary16 weights whatever the scales (the _x kernels).
+// EXACT: the weights are formed in two exact parts (decode_frag_split) for any int8
+// scale: three matrix-core products per k-step instead of two (the _x kernels).  The
+// split of the scale into 16 sh + sl that this replaced took four: a block of the model
+// with whole-range scales at 7 / 64 / 512 / 1500 / 3000 tokens 596 / 588 / 1392 / 3165 /
+// 5266 us with four, 570 / 548 / 1286 / 2688 / 4440 us with three; error against 64-bit
+// arithmetic the same (the rest r xl is 2e-8 of a sum over uniform scales and codes).
 template <bool PAIR, int NJ, bool EXACT = false>
 __device__ __forceinline__ void gemm_body(const GemmArgs &a)
 {
@@ -1007,22 +1020,21 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
             }
         }
         } else {
-        SplitScales sp[2][2];
+        half2v ss[2][2];
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int ch = 0; ch < 2; ++ch)
-                sp[i][ch] = stage_scales_split(A[i][ch].sc, q);
-        half8 afh[2], afl[2];
+                ss[i][ch] = stage_scales(A[i][ch].sc, q).sc;
+        SplitFrag afc[2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            afh[i] = decode_frag(A[i][0], 2 * q, sp[i][0].sh);
-            afl[i] = decode_frag(A[i][0], 2 * q, sp[i][0].sl);
-        }
+        for (int i = 0; i < 2; ++i)
+            afc[i] = decode_frag_split(A[i][0], 2 * q, ss[i][0][0]);
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const uint32_t kp = ks * 2 + p;
-            half8 anh[2], anl[2], bfh[2], bfl[2];
+            half8 bfh[2], bfl[2];
+            SplitFrag afn[2];
             bfh[0] = lds_frag(bh, swz(lr, kp));
             bfl[0] = lds_frag(bl, swz(lr, kp));
 #pragma unroll
@@ -1032,30 +1044,25 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
                     bfl[(j + 1) & 1] = lds_frag(bl, swz((j + 1) * 32 + lr, kp));
                 }
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afh[i], bfh[j & 1], acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afl[i], bfh[j & 1], acc[i][j], 0, 0, 0);
-                }
+                for (int i = 0; i < 2; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].w, bfh[j & 1], acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].r, bfh[j & 1], acc[i][j], 0, 0, 0);
                 if (j == 1 && ks < 3) {
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        const SplitScales &n = sp[i][(ks + 1) & 1];
-                        anh[i] = decode_frag(A[i][(ks + 1) & 1], 2 * q + ((ks + 1) >> 1), n.sh);
-                        anl[i] = decode_frag(A[i][(ks + 1) & 1], 2 * q + ((ks + 1) >> 1), n.sl);
-                    }
+                    for (int i = 0; i < 2; ++i)
+                        afn[i] = decode_frag_split(A[i][(ks + 1) & 1], 2 * q + ((ks + 1) >> 1),
+                                                   ss[i][(ks + 1) & 1][((ks + 1) >> 1) & 1]);
                 }
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afh[i], bfl[j & 1], acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afl[i], bfl[j & 1], acc[i][j], 0, 0, 0);
-                }
+                for (int i = 0; i < 2; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].w, bfl[j & 1], acc[i][j], 0, 0, 0);
             }
             if (ks < 3) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    afh[i] = anh[i];
-                    afl[i] = anl[i];
-                }
+                for (int i = 0; i < 2; ++i)
+                    afc[i] = afn[i];
             }
         }
         }
@@ -1162,8 +1169,8 @@ k_gemm_q6_swiglu(const GemmArgs a)
     gemm_body<true, 4>(a);
 }
 
-// Split-scale forms (weights with some |sc| > 64): 64 token columns per workgroup,
-// so that the second set of weight fragments fits the registers.
+// Two-part weights (some |sc| > 64): 64 token columns per workgroup, so that the second
+// set of weight fragments fits the registers.
 extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 k_gemm_q6_x(const GemmArgs a)
 {
@@ -1411,7 +1418,7 @@ k_gemm_swiglu_h16(const GemmArgs a)
 // so there is no LDS tile and no barrier, and each wave waits only for the
 // loads its next instructions use.  Same arithmetic per (row, token) as
 // gemm_body.  NI: 32-row tiles per wave (the pair form: its gate and up tile).
-// EXACT: split-scale weights as in gemm_body (the _x kernels).
+// EXACT: weights in two parts as in gemm_body (the _x kernels).
 template <bool PAIR, int NI, int G, bool EXACT = false>
 __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
 {
@@ -1625,46 +1632,39 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
             }
         }
         } else {
-        half8 afh[NI], afl[NI];
-        SplitScales sp[NI][2];
+        SplitFrag afc[NI];
+        half2v ss[NI][2];
 #pragma unroll
         for (int i = 0; i < NI; ++i)
 #pragma unroll
             for (int ch = 0; ch < 2; ++ch)
-                sp[i][ch] = stage_scales_split(A[i][ch].sc, q);
+                ss[i][ch] = stage_scales(A[i][ch].sc, q).sc;
 #pragma unroll
-        for (int i = 0; i < NI; ++i) {
-            afh[i] = decode_frag(A[i][0], 2 * q, sp[i][0].sh);
-            afl[i] = decode_frag(A[i][0], 2 * q, sp[i][0].sl);
-        }
+        for (int i = 0; i < NI; ++i)
+            afc[i] = decode_frag_split(A[i][0], 2 * q, ss[i][0][0]);
         lds_frags_wait(bch, bcl);
 #pragma unroll
         for (int kq = 0; kq < 4; ++kq) {
-            half8 anh[NI], anl[NI];
+            SplitFrag afn[NI];
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afh[i], bch[kq], acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afl[i], bch[kq], acc[i], 0, 0, 0);
-            }
+            for (int i = 0; i < NI; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].w, bch[kq], acc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].r, bch[kq], acc[i], 0, 0, 0);
             if (kq < 3) {
 #pragma unroll
-                for (int i = 0; i < NI; ++i) {
-                    const SplitScales &n = sp[i][(kq + 1) & 1];
-                    anh[i] = decode_frag(A[i][(kq + 1) & 1], 2 * q + ((kq + 1) >> 1), n.sh);
-                    anl[i] = decode_frag(A[i][(kq + 1) & 1], 2 * q + ((kq + 1) >> 1), n.sl);
-                }
+                for (int i = 0; i < NI; ++i)
+                    afn[i] = decode_frag_split(A[i][(kq + 1) & 1], 2 * q + ((kq + 1) >> 1),
+                                               ss[i][(kq + 1) & 1][((kq + 1) >> 1) & 1]);
             }
 #pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afh[i], bcl[kq], acc[i], 0, 0, 0);
-                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afl[i], bcl[kq], acc[i], 0, 0, 0);
-            }
+            for (int i = 0; i < NI; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].w, bcl[kq], acc[i], 0, 0, 0);
             if (kq < 3) {
 #pragma unroll
-                for (int i = 0; i < NI; ++i) {
-                    afh[i] = anh[i];
-                    afl[i] = anl[i];
-                }
+                for (int i = 0; i < NI; ++i)
+                    afc[i] = afn[i];
             }
         }
         }
@@ -1857,7 +1857,7 @@ extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_t32n1(const Gem
     gemm_small_body<false, 1, 2>(a); // three workgroups per CU: 6 tile buffers fit their LDS
 }
 
-// Split-scale forms (weights with some |sc| > 64): one 32-row tile per wave for
+// Two-part weights (some |sc| > 64): one 32-row tile per wave for
 // single weights, the gate and up tiles for the pair.
 extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_t32x(const GemmArgs a)
 {
