@@ -272,11 +272,13 @@ struct SplitArgs {
     float *logit_out;    // nullable: the router logits [T][n_expert] (routing log)
     uint32_t nparts;
     // nullable (small calls): before the split, row t of x first gets the down
-    // projection's ranks combined into it as k_reduce_combine does (x += sum_r
+    // projection's ranks combined into it (x += sum_r
     // cwsel[t][r] (sum_s cpart[s][t*4 + r]), rank then slice order), written back
+    // (a slice of cpart holds crows token rows: T, or more when the split takes the
+    // last T rows of the call)
     const float *cpart, *cwsel;
     float *cx;
-    uint32_t cksplit, cn_used;
+    uint32_t cksplit, cn_used, crows;
     // nullable: the workgroups also copy copy_n floats (a multiple of 4, 16-byte
     // aligned) from copy_src to copy_dst (the short conv's new state, written by the
     // kernel before this one)
@@ -391,13 +393,6 @@ struct GemmReduceArgs {    // c (+)= sum_s part[s] in slice order; pair: silu(g)
     uint32_t *counts; // nullable (with rw): workgroup (0, 0) zeroes counts[0 .. n_expert)
 };
 
-struct ReduceCombineArgs { // x[t] += sum_r w[t][r] * (sum_s part[s][t*4 + r]), rank then slice order
-    const float *part;       // [ksplit][T*4][dim]
-    const float *wsel;       // [T][4]
-    float *x;                // [T][dim]
-    uint32_t ksplit, T, dim, n_used;
-};
-
 struct ConvPrefillArgs {  // gated short conv over T tokens, parallel in t
     const float *bcx;     // [ksplit][T][3*dim] in_proj rows B, C, X (ksplit > 1: the
                           // split-K partial sums, added here in slice order)
@@ -406,6 +401,8 @@ struct ConvPrefillArgs {  // gated short conv over T tokens, parallel in t
     float *state_next;    // [dim][2] after it (copied over `state` by the next split)
     float *y;             // [T][dim]
     uint32_t T, dim, ksplit;
+    uint32_t t0;          // the grid covers tokens t0 .. T - 1; when that is T - 1 alone,
+                          // state_next may be state (each thread reads and writes its own)
     // nullable (small calls): y stored binary16 hi + lo in the blocked layout (logical
     // row t, width dim) with the power-of-two scale of each 128 channels' largest
     // magnitude at y_bscale[t * (dim / 128) + ch / 128], instead of fp32 in y, so

@@ -177,7 +177,7 @@ __device__ __forceinline__ void split_pieces(const SplitArgs &a, uint32_t t, flo
     }
 }
 
-// Row t of x plus the down projection's ranks, as k_reduce_combine forms it:
+// Row t of x plus the down projection's ranks:
 // d_r = sum of the cksplit slices in slice order, then x + ((0 + d_0 w_0) + d_1 w_1
 // ...) over the used ranks (lfm.rs:645-668, no contraction); the new values are
 // written back to cx.  v holds the row's pieces (thread tid: pieces tid + 256 i).
@@ -185,7 +185,7 @@ __device__ __forceinline__ void combine_pieces(const SplitArgs &a, uint32_t t, f
 {
 #pragma clang fp contract(off)
     const uint32_t tid = threadIdx.x, npc = a.K >> 3;
-    const size_t D = a.K, slice = (size_t)a.T * 4 * D;
+    const size_t D = a.K, slice = (size_t)a.crows * 4 * D;
     float w[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -1966,7 +1966,7 @@ extern "C" __global__ __launch_bounds__(WG_THREADS) void k_conv_prefill(const Co
 {
 #pragma clang fp contract(off)
     const uint32_t ch = blockIdx.x * WG_THREADS + threadIdx.x;
-    const uint32_t t = blockIdx.y;
+    const uint32_t t = a.t0 + blockIdx.y;
     if (ch >= a.dim || t >= a.T)
         return;
     const size_t D3 = 3 * (size_t)a.dim, slice = (size_t)a.T * D3;
@@ -2566,33 +2566,6 @@ extern "C" __global__ __launch_bounds__(WG_THREADS) void k_combine_prefill(const
             sm.w = sm.w + dv[r].w * wv[r];
         }
     *xp = make_float4(x0.x + sm.x, x0.y + sm.y, x0.z + sm.z, x0.w + sm.w);
-}
-
-// The expert down projection's K slices and the combine in one pass (split-K
-// calls): d = sum_s part[s] in slice order, then k_combine_prefill's
-// x += ((0 + d_0 w_0) + d_1 w_1) + ... in rank order, no contraction.
-extern "C" __global__ __launch_bounds__(WG_THREADS) void k_reduce_combine(const ReduceCombineArgs a)
-{
-#pragma clang fp contract(off)
-    const uint32_t k = blockIdx.x * WG_THREADS + threadIdx.x, t = blockIdx.y;
-    if (k >= a.dim || t >= a.T)
-        return;
-    const size_t slice = (size_t)a.T * 4 * a.dim;
-    float *x = a.x + (size_t)t * a.dim + k;
-    const float x0 = *x;
-    float w[4], d[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-        w[r] = a.wsel[(size_t)t * 4 + r];
-    // the four ranks' slices together (ranks >= n_used are read and not used)
-    const size_t D = a.dim;
-    slice_sums<4>(a.part + (size_t)t * 4 * a.dim + k, slice, a.ksplit, {0, D, 2 * D, 3 * D}, d);
-    float sm = 0.0f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-        if (r < (int)a.n_used)
-            sm = sm + d[r] * w[r];
-    *x = x0 + sm;
 }
 
 // Token embeddings of T ids (lfm.rs:310-320): row ids[t] of the Q6_K table,
