@@ -114,7 +114,8 @@ struct Kernels {
         tile_pack, gemm_q6_n64, gemm_q6_x, gemm_swiglu_x, gemm_q6_t32x, gemm_swiglu_t32x, tile_h16, gemm_h16,
         gemm_h16_n64, gemm_swiglu_h16;
     hipFunction_t matvec_long, attn, attn_merge, router, moe_down, argmax, argmax_final, advance,
-        dequant, copy, matvec_route, gateup_f, conv_mixer, conv_mixer_r, session_out, session_in;
+        dequant, copy, matvec_route, gateup_f, conv_mixer, conv_mixer_r, session_out, session_in, conv_clear, start,
+        host_out;
     Shape matvec, conv, qkv, gateup, head;
     DevState *idle_st = nullptr; // zeroed state for op-level matvecs (never halted)
 };
@@ -217,7 +218,8 @@ static int get_kernels(Kernels **out)
                {&k->dequant, "k_q6_dequant"},    {&k->copy, "k_copy"},
                {&k->matvec_route, "k_q6_matvec_route"}, {&k->gateup_f, "k_gateup8f"},
                {&k->conv_mixer, "k_conv_mixer"},  {&k->conv_mixer_r, "k_conv_mixer_r"},
-               {&k->session_out, "k_session_out"}, {&k->session_in, "k_session_in"}};
+               {&k->session_out, "k_session_out"}, {&k->session_in, "k_session_in"},
+               {&k->conv_clear, "k_conv_clear"}, {&k->start, "k_start"}, {&k->host_out, "k_host_out"}};
     for (auto &f : fns) {
         e = hipModuleGetFunction(f.f, k->mod, f.name);
         if (e != hipSuccess) {
@@ -860,7 +862,7 @@ int lfm_argmax_enqueue(const float *v, uint32_t n, DevState *st, float *partial,
     RC(get_kernels(&K));
     const uint32_t grid = lfm_argmax_grid(n);
     ArgmaxArgs a{v, partial, n, st};
-    FinalArgs f{partial, grid, nullptr, 0, st, nullptr};
+    FinalArgs f{partial, grid, nullptr, 0, st, nullptr, nullptr, nullptr, 0};
     RC(launch(K->argmax, dim3(grid), 0, s, a));
     return launch(K->argmax_final, dim3(1), 0, s, f);
 }
@@ -957,7 +959,6 @@ struct lfm_engine {
     std::vector<float *> conv;
     uint32_t head_grid = 1, nchunk = 1;
     float *rope = nullptr; // [ctx][32] (cos, sin)
-    DevState *host_st = nullptr;    // pinned staging for state copies
     HostResult *host_res = nullptr; // pinned, device-mapped: forward calls' results
     HostResult *host_res_dev = nullptr; // its device address
     // session copies: SESSION_SLOTS pinned chunks, their device address, and the
@@ -990,7 +991,10 @@ struct lfm_engine {
         // small calls: the conv state the next split moves from cstate into place
         float *state_pending = nullptr;
     } pf;
-    uint32_t *host_ids = nullptr;   // pinned staging for prompt ids (ctx entries)
+    // pinned, device-mapped: a call's prompt ids (ctx entries), read by the embedding
+    // launch, and what a call returns (logits, or the decode state and the tokens)
+    uint32_t *host_ids = nullptr, *host_ids_dev = nullptr;
+    uint32_t *host_out = nullptr, *host_out_dev = nullptr;
 
     // conv mixers of the captured step in one launch each (k_conv_mixer*): the
     // gated output's tagged entries, and whether the grid fits co-resident
@@ -1465,9 +1469,14 @@ static int enq_ffn(lfm_engine *e, uint32_t l, bool fuse, float *x = nullptr, uin
     return LFM_OK;
 }
 
+// Workgroups that store n words to pinned host memory: one 16-byte unit per thread.
+static uint32_t host_out_grid(uint32_t n) { return std::min(256u, std::max(1u, (n + 1023) / 1024)); }
+
 // x: the residual to finish (the decode state's e->x, or a prefill's last row);
-// host: nullable device address of pinned memory that also receives the result.
-static int enq_head(lfm_engine *e, uint32_t advance, const float *x = nullptr, HostResult *host = nullptr)
+// host: nullable device address of pinned memory that also receives the result;
+// logits: the logits go to e->host_out too.
+static int enq_head(lfm_engine *e, uint32_t advance, const float *x = nullptr, HostResult *host = nullptr,
+                    bool logits = false)
 {
     HeadArgs h;
     h.emb = q6(e, "token_embd.weight");
@@ -1477,8 +1486,8 @@ static int enq_head(lfm_engine *e, uint32_t advance, const float *x = nullptr, H
     h.vocab = e->hp.vocab;
     h.st = e->st;
     RC(launch_t(e->K->head.fn(), dim3(e->head_grid), e->K->head.threads(), 0, e->stream, h));
-    FinalArgs f{e->hpart, e->head_grid, e->out_tokens, advance, e->st, host};
-    RC(launch(e->K->argmax_final, dim3(1), 0, e->stream, f));
+    FinalArgs f{e->hpart, e->head_grid, e->out_tokens, advance, e->st, host, e->logits, (float *)e->host_out_dev, e->hp.vocab};
+    RC(launch(e->K->argmax_final, dim3(logits ? 1 + host_out_grid(e->hp.vocab) : 1), 0, e->stream, f));
     e->dispatches += 2;
     return LFM_OK;
 }
@@ -1606,8 +1615,7 @@ extern "C" int lfm_engine_finalize(lfm_engine *e)
         HIPCHK(hipMemcpy(e->rope, tab.data(), tab.size() * 4, hipMemcpyHostToDevice));
     }
     const size_t swn = std::max<size_t>((size_t)hp.n_ff, (size_t)hp.n_used * hp.expert_ff);
-    HIPCHK(hipHostMalloc((void **)&e->host_st, sizeof(DevState), hipHostMallocDefault));
-    // forward calls' results, stored by the last kernel into host memory
+    // calls' results, stored by their last kernel into host memory
     HIPCHK(hipHostMalloc((void **)&e->host_res, sizeof(HostResult), hipHostMallocCoherent | hipHostMallocMapped));
     HIPCHK(hipHostGetDevicePointer((void **)&e->host_res_dev, e->host_res, 0));
     HIPCHK(hipHostMalloc((void **)&e->session_buf, (size_t)SESSION_SLOTS * SESSION_CHUNK * 4,
@@ -1615,7 +1623,11 @@ extern "C" int lfm_engine_finalize(lfm_engine *e)
     HIPCHK(hipHostGetDevicePointer((void **)&e->session_dev, e->session_buf, 0));
     for (hipEvent_t &ev : e->session_ev)
         HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    HIPCHK(hipHostMalloc((void **)&e->host_ids, (size_t)e->ctx * 4, hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void **)&e->host_ids, (size_t)e->ctx * 4, hipHostMallocCoherent | hipHostMallocMapped));
+    HIPCHK(hipHostGetDevicePointer((void **)&e->host_ids_dev, e->host_ids, 0));
+    const size_t out_words = std::max<size_t>(hp.vocab, DEV_STATE_WORDS + (size_t)e->ctx);
+    HIPCHK(hipHostMalloc((void **)&e->host_out, out_words * 4, hipHostMallocCoherent | hipHostMallocMapped));
+    HIPCHK(hipHostGetDevicePointer((void **)&e->host_out_dev, e->host_out, 0));
     HIPCHK(hipMalloc(&e->st, sizeof(DevState)));
     HIPCHK(hipMemset(e->st, 0, sizeof(DevState)));
     HIPCHK(hipMalloc(&e->ids, e->ctx * 4));
@@ -1825,8 +1837,6 @@ extern "C" void lfm_engine_destroy(lfm_engine *e)
     for (void *p : bufs)
         if (p)
             (void)hipFree(p);
-    if (e->host_st)
-        (void)hipHostFree(e->host_st);
     if (e->host_res)
         (void)hipHostFree(e->host_res);
     if (e->session_buf)
@@ -1836,6 +1846,8 @@ extern "C" void lfm_engine_destroy(lfm_engine *e)
             (void)hipEventDestroy(ev);
     if (e->host_ids)
         (void)hipHostFree(e->host_ids);
+    if (e->host_out)
+        (void)hipHostFree(e->host_out);
     for (auto p : e->qkvdev)
         if (p)
             (void)hipFree(p);
@@ -2277,11 +2289,11 @@ static int pf_ffn(lfm_engine *e, uint32_t l, uint32_t T)
     return LFM_OK;
 }
 
-// Runs the layer stack for e->ids[0..T) at positions start.. and leaves the
-// last token's residual in row T - 1 of pf.x.
-// ids (nullable, T <= EMBED_INLINE_IDS): the call's ids, passed in the embedding
-// launch's arguments, which also starts the decode state (no copies before it).
-static int enq_prefill(lfm_engine *e, uint32_t T, uint32_t start, const uint32_t *ids = nullptr)
+// Runs the layer stack for the ids at positions start.. and leaves the last token's
+// residual in row T - 1 of pf.x.  No copy precedes the first kernel: the embedding
+// launch starts the decode state and takes up to EMBED_INLINE_IDS ids in its
+// arguments, more from pinned host memory (no earlier work may still read it).
+static int enq_prefill(lfm_engine *e, uint32_t T, uint32_t start, const uint32_t *ids)
 {
     const lfm_hparams &hp = e->hp;
     if (e->route_log)
@@ -2291,16 +2303,15 @@ static int enq_prefill(lfm_engine *e, uint32_t T, uint32_t start, const uint32_t
     EmbedRowsArgs em;
     memset(&em, 0, sizeof(em));
     em.emb = q6(e, "token_embd.weight");
-    em.ids = e->ids;
     em.x = e->pf.x;
     em.T = T;
-    if (ids) {
-        if (T > EMBED_INLINE_IDS)
-            return fail(LFM_EINTERNAL, "prefill: %u inline ids > %u", T, EMBED_INLINE_IDS);
-        em.ids = nullptr;
+    em.st = e->st;
+    em.start = start;
+    if (T <= EMBED_INLINE_IDS) {
         memcpy(em.ids_inline, ids, (size_t)T * 4);
-        em.st = e->st;
-        em.start = start;
+    } else {
+        memcpy(e->host_ids, ids, (size_t)T * 4);
+        em.ids = e->host_ids_dev;
     }
     RC(launch(e->K->embed_rows, dim3((T + 3) / 4), 0, e->stream, em));
     e->dispatches += 1;
@@ -2325,33 +2336,34 @@ static int need_final(lfm_engine *e)
     return LFM_OK;
 }
 
-// Writes the device-resident decode state.
+// Starts the device-resident decode state.
 static int set_state(lfm_engine *e, uint32_t tok, uint32_t pos, uint32_t n_ids, uint32_t eos)
 {
-    HIPCHK(hipStreamSynchronize(e->stream)); // the pinned staging block is reused
-    DevState &h = *e->host_st;
-    memset(&h, 0, sizeof(h));
-    h.tok = tok;
-    h.pos = pos;
-    h.halt = 0;
-    h.step = 0;
-    h.eos = eos;
-    h.cursor = 0;
-    h.n_ids = n_ids;
-    // everything but the step generation, which only the device advances
-    HIPCHK(hipMemcpyAsync(e->st, &h, offsetof(DevState, gen), hipMemcpyHostToDevice, e->stream));
+    const StartArgs a{e->st, tok, pos, n_ids, eos};
+    RC(launch_t(e->K->start, dim3(1), 64, 0, e->stream, a));
+    e->dispatches += 1;
     return LFM_OK;
 }
 
-// Reads the device state back after the stream's work; a fused kernel's
-// bounded handoff wait that timed out (the grid was not co-resident) fails the
-// call that ran it.
-static int read_state(lfm_engine *e, DevState *h)
+// Waits for the stream's work and two runs of device words (16-byte aligned) after it
+// in e->host_out, stored there by a kernel.  (hipMemcpy to the caller's pageable memory
+// is a kernel into a staging buffer, a wait and a host copy, once per copy: a token
+// with its logits at position 2900 of a 4-layer block of the model took 192 us with
+// state, ids, logits and result copied, 161 us with none.)
+static int host_out(lfm_engine *e, const void *a, uint32_t na, const void *b = nullptr, uint32_t nb = 0)
 {
-    HIPCHK(hipMemcpyAsync(e->host_st, e->st, sizeof(DevState), hipMemcpyDeviceToHost, e->stream));
+    const HostOutArgs o{(const uint32_t *)a, (const uint32_t *)b, na, nb, e->host_out_dev};
+    RC(launch(e->K->host_out, dim3(host_out_grid(na + nb)), 0, e->stream, o));
+    e->dispatches += 1;
     HIPCHK(hipStreamSynchronize(e->stream));
-    *h = *e->host_st;
-    if (h->fault)
+    return LFM_OK;
+}
+
+// A fused kernel's bounded handoff wait that timed out (the grid was not co-resident)
+// fails the call that ran it.
+static int check_fault(uint32_t fault)
+{
+    if (fault)
         return fail(LFM_EDEVICE, "a fused decode kernel's handoff wait timed out (workgroups not co-resident)");
     return LFM_OK;
 }
@@ -2370,32 +2382,31 @@ static int check_ids(lfm_engine *e, const uint32_t *ids, uint32_t n, uint32_t st
 
 static_assert(LFM_MAX_TOKEN_BATCH <= EMBED_INLINE_IDS, "forward_token batches fit the embedding launch's ids");
 
-// Layers for every id (graph replays), then the head without feedback; the
-// result also goes to the pinned e->host_res.
-static int run_prompt(lfm_engine *e, const uint32_t *ids, uint32_t n, uint32_t start)
+// Layers for every id (one matrix-core call, or graph replays), then the head without
+// feedback.  Returns with the stream's work done and its result in e->host_res, with
+// the logits in e->host_out when `logits` is set.
+static int run_prompt(lfm_engine *e, const uint32_t *ids, uint32_t n, uint32_t start, bool logits)
 {
     RC(check_ids(e, ids, n, start));
-    e->host_res->token = ~0u; // every earlier call has synchronized: no kernel writes it now
+    HIPCHK(hipStreamSynchronize(e->stream)); // a call that failed part-way: the pinned blocks are reused
     const bool prefill = n >= 2 && !e->stepwise_prefill;
-    if (prefill && n <= EMBED_INLINE_IDS) {
-        // forward_token batches: the ids travel in the embedding launch's arguments,
-        // which also starts the decode state (no copies ahead of the first kernel)
+    if (prefill) {
         RC(enq_prefill(e, n, start, ids));
     } else {
-        RC(set_state(e, ids[0], start, n, 0xFFFFFFFFu)); // also waits for prior use of host_ids
-        memcpy(e->host_ids, ids, (size_t)n * 4);
-        HIPCHK(hipMemcpyAsync(e->ids, e->host_ids, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
-        if (prefill) {
-            RC(enq_prefill(e, n, start)); // matrix-core path
-        } else {
-            for (uint32_t j = 0; j < n; ++j) { // one captured decode step per token
-                HIPCHK(hipGraphLaunch(e->g_layers, e->stream));
-                e->dispatches += e->nodes_layers;
-            }
+        RC(set_state(e, ids[0], start, n, 0xFFFFFFFFu));
+        if (n > 1) { // k_advance takes the later ids
+            memcpy(e->host_ids, ids, (size_t)n * 4);
+            HIPCHK(hipMemcpyAsync(e->ids, e->host_ids, (size_t)n * 4, hipMemcpyHostToDevice, e->stream));
+        }
+        for (uint32_t j = 0; j < n; ++j) { // one captured decode step per token
+            HIPCHK(hipGraphLaunch(e->g_layers, e->stream));
+            e->dispatches += e->nodes_layers;
         }
     }
-    RC(enq_head(e, 0, prefill ? e->pf.x + (size_t)(n - 1) * e->hp.dim : e->x, e->host_res_dev));
-    return LFM_OK;
+    RC(enq_head(e, 0, prefill ? e->pf.x + (size_t)(n - 1) * e->hp.dim : e->x, e->host_res_dev, logits));
+    HIPCHK(hipStreamSynchronize(e->stream));
+    // (the state started unhalted and no kernel of a prompt halts it: the result is there)
+    return check_fault(e->host_res->fault);
 }
 
 extern "C" int lfm_forward_logits(lfm_engine *e, const uint32_t *ids, uint32_t n, uint32_t start,
@@ -2404,11 +2415,9 @@ extern "C" int lfm_forward_logits(lfm_engine *e, const uint32_t *ids, uint32_t n
     RC(need_final(e));
     if (!logits || cap < e->hp.vocab)
         return fail(LFM_ERANGE, "logits buffer holds %zu < vocab %u floats", cap, e->hp.vocab);
-    RC(run_prompt(e, ids, n, start));
-    HIPCHK(hipMemcpyAsync(logits, e->logits, (size_t)e->hp.vocab * 4, hipMemcpyDeviceToHost,
-                          e->stream));
-    DevState h;
-    return read_state(e, &h);
+    RC(run_prompt(e, ids, n, start, true));
+    memcpy(logits, e->host_out, (size_t)e->hp.vocab * 4);
+    return LFM_OK;
 }
 
 extern "C" int lfm_forward_token(lfm_engine *e, const uint32_t *ids, uint32_t n, uint32_t start,
@@ -2419,23 +2428,10 @@ extern "C" int lfm_forward_token(lfm_engine *e, const uint32_t *ids, uint32_t n,
         return fail(LFM_EINVAL, "token batch must be 1..%d", LFM_MAX_TOKEN_BATCH);
     if (!next)
         return fail(LFM_EINVAL, "next is null");
-    RC(run_prompt(e, ids, n, start));
-    HIPCHK(hipStreamSynchronize(e->stream));
-    const HostResult r = *e->host_res; // written by k_argmax_final (no copy back)
-    if (r.token == ~0u) // not stored (a halted state): the state copy has the result
-    {
-        DevState h;
-        RC(read_state(e, &h));
-        *next = h.last_token;
-        if (max_logit)
-            *max_logit = h.last_value;
-        return LFM_OK;
-    }
-    if (r.fault)
-        return fail(LFM_EDEVICE, "a fused decode kernel's handoff wait timed out (workgroups not co-resident)");
-    *next = r.token;
+    RC(run_prompt(e, ids, n, start, false));
+    *next = e->host_res->token;
     if (max_logit)
-        *max_logit = r.value;
+        *max_logit = e->host_res->value;
     return LFM_OK;
 }
 
@@ -2467,10 +2463,12 @@ extern "C" int lfm_decode_run(lfm_engine *e, uint32_t first, uint32_t start, uin
         HIPCHK(hipGraphLaunch(e->g_decode, e->stream));
         e->dispatches += e->nodes_decode;
     }
+    RC(host_out(e, e->st, DEV_STATE_WORDS, e->out_tokens, steps));
     DevState h;
-    RC(read_state(e, &h));
+    memcpy(&h, e->host_out, sizeof(h));
+    RC(check_fault(h.fault));
     const uint32_t n = std::min(h.step, steps);
-    HIPCHK(hipMemcpy(out_tokens, e->out_tokens, (size_t)n * 4, hipMemcpyDeviceToHost));
+    memcpy(out_tokens, e->host_out + DEV_STATE_WORDS, (size_t)n * 4);
     *n_out = n;
     return LFM_OK;
 }
@@ -2478,9 +2476,16 @@ extern "C" int lfm_decode_run(lfm_engine *e, uint32_t first, uint32_t start, uin
 extern "C" int lfm_reset_session(lfm_engine *e)
 {
     RC(need_final(e));
+    SessionArgs a;
+    memset(&a, 0, sizeof(a));
+    a.count = e->hp.dim * 2; // dim is a multiple of 256
     for (uint32_t l = 0; l < e->hp.n_layers; ++l)
         if (e->conv[l])
-            HIPCHK(hipMemsetAsync(e->conv[l], 0, (size_t)e->hp.dim * 2 * 4, e->stream));
+            a.seg[a.nseg++] = SessionSeg{e->conv[l], 0, 0};
+    if (a.nseg) {
+        RC(launch(e->K->conv_clear, dim3((a.count + 1023) / 1024, a.nseg), 0, e->stream, a));
+        e->dispatches += 1;
+    }
     HIPCHK(hipStreamSynchronize(e->stream));
     return LFM_OK;
 }
@@ -2635,8 +2640,8 @@ extern "C" int lfm_snapshot_logits(lfm_engine *e, float *out, size_t cap)
     RC(need_final(e));
     if (!out || cap < e->hp.vocab)
         return fail(LFM_ERANGE, "logits buffer holds %zu < vocab %u floats", cap, e->hp.vocab);
-    HIPCHK(hipStreamSynchronize(e->stream));
-    HIPCHK(hipMemcpy(out, e->logits, (size_t)e->hp.vocab * 4, hipMemcpyDeviceToHost));
+    RC(host_out(e, e->logits, e->hp.vocab));
+    memcpy(out, e->host_out, (size_t)e->hp.vocab * 4);
     return LFM_OK;
 }
 

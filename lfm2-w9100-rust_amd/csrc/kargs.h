@@ -36,6 +36,30 @@ struct DevState {
                         // the host never rewrites it (fused kernels' handoff tags)
 };                      // 64 bytes
 static_assert(sizeof(DevState) == 64, "DevState is 64 bytes");
+#define DEV_STATE_WORDS 16
+
+// Starts a call's decode state: everything but gen, which only the last kernel of a
+// step advances.  One thread of the call's first kernel runs it.
+__device__ inline void start_state(DevState *st, uint32_t tok, uint32_t pos, uint32_t n_ids, uint32_t eos)
+{
+    st->tok = tok;
+    st->pos = pos;
+    st->halt = 0;
+    st->step = 0;
+    st->eos = eos;
+    st->cursor = 0;
+    st->n_ids = n_ids;
+    st->last_token = 0;
+    st->last_value = 0.f;
+    st->fault = 0;
+    for (int i = 0; i < 5; ++i)
+        st->pad[i] = 0;
+}
+
+struct StartArgs {
+    DevState *st;
+    uint32_t tok, pos, n_ids, eos;
+};
 
 // Where a kernel's input vector comes from.
 struct XSrc {
@@ -199,6 +223,17 @@ struct FinalArgs {       // reduce partials; decode step: store, feed back, adva
     uint32_t advance;
     DevState *st;
     HostResult *host;    // nullable: also store the result here (device address of pinned memory)
+    // nullable: workgroups 1 .. also copy the n_logits logits to this pinned memory
+    const float *logits;
+    float *logits_host;
+    uint32_t n_logits;
+};
+
+// Two runs of device words stored to pinned host memory, b after a.
+struct HostOutArgs {
+    const uint32_t *a, *b;
+    uint32_t na, nb;
+    uint32_t *host;
 };
 
 struct AdvanceArgs {
@@ -498,13 +533,10 @@ struct CombinePrefillArgs {  // x[t] += sum_r w[t][r] * D[t*4 + r] (rank order)
 #define EMBED_INLINE_IDS 64 // forward_token's batch limit
 struct EmbedRowsArgs {
     Q6T emb;
-    const uint32_t *ids;  // [T]; null: ids_inline (T <= EMBED_INLINE_IDS)
+    const uint32_t *ids;  // [T], pinned host memory; null: ids_inline (T <= EMBED_INLINE_IDS)
     float *x;             // [T][dim]
     uint32_t T;
-    // nullable: workgroup 0 also starts the call's decode state (the host's
-    // set_state without a copy): tok = the first id, pos = start, eos = ~0u,
-    // n_ids = T, the other fields but gen zero
-    DevState *st;
+    DevState *st;         // workgroup 0 also starts the call's decode state
     uint32_t start;
     uint32_t ids_inline[EMBED_INLINE_IDS];
 };
@@ -520,6 +552,7 @@ struct SessionSeg {
 };
 struct SessionArgs {
     float *host; // device address of pinned host memory: float `first` at host[0]
+                 // (k_conv_clear: unused, first 0, every segment a conv state of count floats)
     uint32_t first, count, nseg, ctx;
     SessionSeg seg[SESSION_SEGS];
 };

@@ -1452,12 +1452,44 @@ extern "C" __global__ __launch_bounds__(WG_THREADS) void k_argmax(const ArgmaxAr
     }
 }
 
+// n device words stored to pinned host memory (16-byte aligned both), workgroup wg of
+// nwg: consecutive threads on consecutive 16-byte units.
+__device__ __forceinline__ void store_host(uint32_t *host, const uint32_t *dev, uint32_t n, uint32_t wg, uint32_t nwg)
+{
+    const uint32_t n4 = n / 4;
+    for (uint32_t i = wg * WG_THREADS + threadIdx.x; i < n4; i += nwg * WG_THREADS)
+        reinterpret_cast<uint4 *>(host)[i] = reinterpret_cast<const uint4 *>(dev)[i];
+    if (wg == 0 && threadIdx.x < n - 4 * n4)
+        host[4 * n4 + threadIdx.x] = dev[4 * n4 + threadIdx.x];
+}
+
+// Starts the decode state of a call that does not go through the embedding launch.
+extern "C" __global__ void k_start(const StartArgs a)
+{
+    if (threadIdx.x == 0)
+        start_state(a.st, a.tok, a.pos, a.n_ids, a.eos);
+}
+
+// Results of a call for the host to read once the stream has synchronized.
+extern "C" __global__ __launch_bounds__(WG_THREADS) void k_host_out(const HostOutArgs a)
+{
+    store_host(a.host, a.a, a.na, blockIdx.x, gridDim.x);
+    store_host(a.host + a.na, a.b, a.nb, blockIdx.x, gridDim.x);
+}
+
 // Reduces the partials; in a decode step stores the token and feeds it back
-// (stops the loop at eos, main.rs:182-189).
+// (stops the loop at eos, main.rs:182-189).  For a forward call that returns its
+// logits the workgroups after the first store them to pinned host memory meanwhile
+// (256 KB for 65536: bound by the host link).
 extern "C" __global__ __launch_bounds__(WG_THREADS) void k_argmax_final(const FinalArgs a)
 {
     if (a.st->halt)
         return;
+    if (blockIdx.x > 0) {
+        store_host(reinterpret_cast<uint32_t *>(a.logits_host), reinterpret_cast<const uint32_t *>(a.logits), a.n_logits,
+                   blockIdx.x - 1, gridDim.x - 1);
+        return;
+    }
     float bv = -INFINITY;
     uint32_t bi = 0;
     for (uint32_t i0 = threadIdx.x; i0 < a.n_partial; i0 += 4 * WG_THREADS) {
@@ -1600,6 +1632,13 @@ extern "C" __global__ __launch_bounds__(256) void k_session_out(const SessionArg
     uint4 *d = reinterpret_cast<uint4 *>(a.host + u);
     d[0] = make_uint4(o[0], o[1], o[2], o[3]);
     d[1] = make_uint4(o[4], o[5], o[6], o[7]);
+}
+// Zeroes the conv states: workgroups (.., s) the count floats of segment s.
+extern "C" __global__ __launch_bounds__(256) void k_conv_clear(const SessionArgs a)
+{
+    const uint32_t u = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (u < a.count)
+        *reinterpret_cast<float4 *>(reinterpret_cast<float *>(a.seg[blockIdx.y].dev) + u) = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 extern "C" __global__ __launch_bounds__(256) void k_session_in(const SessionArgs a)
 {
