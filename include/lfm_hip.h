@@ -244,12 +244,12 @@ int lfm_copy_time(uint64_t bytes, uint32_t reps, float *us_per_copy);
  * multiple of 256 up to 8192 and (T + 31) * in_dim * 2 bytes stays below 2 GiB
  * (the kernels address the binary16 activation copies with 32-bit offsets);
  * LFM_EINVAL otherwise.  This op-level entry point builds its scratch on every
- * call: it allocates the binary16 activation copies, the split-K partial sums
- * (T <= 128) and a 32-row tile copy of the weight (ceil(rows / 32) * in_dim /
- * 256 * 6720 bytes), runs the tile pack kernel, waits for `stream` and frees
- * them, so a caller that loops over it pays for the allocations and the repack
- * each time.  The engine's prefill keeps its
- * tile copies from lfm_engine_finalize and never repacks. */
+ * call and frees it after waiting for `stream`: the binary16 activation copies and
+ * up to 2 MB of split-K partial sums; for T > 1024 also a 32-row tile copy of the
+ * weight (ceil(rows / 32) * in_dim / 256 * 6720 bytes) and, where its scales allow,
+ * a binary16 copy, which a caller that loops over it pays for each time (T <= 1024
+ * reads the packed planes).  The engine's prefill keeps its tile copies from
+ * lfm_engine_finalize and never repacks. */
 int lfm_q6k_gemm(const void *packed_dev, uint64_t rows, uint64_t in_dim, const float *x_dev,
                  uint32_t T, float *y_dev, void *stream);
 

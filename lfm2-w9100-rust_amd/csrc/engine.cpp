@@ -111,7 +111,7 @@ struct Kernels {
     hipModule_t mod = nullptr, pmod = nullptr;
     hipFunction_t split_rows, split_rows_ext, gemm_q6, conv_prefill, rope_kv_prefill, attn_prefill,
         gemm_swiglu, gemm_q6_t32, gemm_q6_t32n1, gemm_swiglu_t32, gemm_reduce, attn_merge_split, router_small, router_mfma, router_split, route_topk, route_group, combine_prefill, embed_rows,
-        tile_pack, gemm_q6_n64, gemm_q6_x, gemm_swiglu_x, gemm_q6_t32x, gemm_swiglu_t32x, tile_h16, gemm_h16,
+        tile_pack, gemm_q6_n64, gemm_q6_x, gemm_swiglu_x, gemm_q6_t32x, gemm_swiglu_t32x, tile_h16, gemm_h16, gemm_q6_rows,
         gemm_h16_n64, gemm_swiglu_h16;
     hipFunction_t matvec_long, attn, attn_merge, router, moe_down, argmax, argmax_final, advance,
         dequant, copy, matvec_route, gateup_f, conv_mixer, conv_mixer_r, session_out, session_in, conv_clear, start,
@@ -253,7 +253,7 @@ static int get_kernels(Kernels **out)
                 {&k->gemm_swiglu_x, "k_gemm_q6_swiglu_x"}, {&k->gemm_q6_t32x, "k_gemm_q6_t32x"},
                 {&k->gemm_swiglu_t32x, "k_gemm_q6_swiglu_t32x"}, {&k->tile_h16, "k_q6_tile_h16"},
                 {&k->gemm_h16, "k_gemm_h16"}, {&k->gemm_h16_n64, "k_gemm_h16_n64"},
-                {&k->gemm_swiglu_h16, "k_gemm_swiglu_h16"}};
+                {&k->gemm_swiglu_h16, "k_gemm_swiglu_h16"}, {&k->gemm_q6_rows, "k_gemm_q6_rows"}};
     for (auto &f : pfns) {
         e = hipModuleGetFunction(f.f, k->pmod, f.name);
         if (e != hipSuccess) {
@@ -471,7 +471,7 @@ static int make_tiles(Kernels *K, hipStream_t s, const Q6T &src, uint32_t group_
         *dev = nullptr;
         return rc;
     }
-    *out = Q6Tiles{(const uint8_t *)*dev, (uint32_t)tiles, src.nb, gtiles, group_rows, wide ? 1u : 0u, nullptr};
+    *out = Q6Tiles{(const uint8_t *)*dev, (uint32_t)tiles, src.nb, gtiles, group_rows, wide ? 1u : 0u, nullptr, 0};
     return LFM_OK;
 }
 
@@ -670,6 +670,11 @@ static bool small_call(uint32_t T, uint32_t dim) { return T <= (dim >= 512 ? SMA
 
 #define GEMM_PART_BYTES ((size_t)64 << 20) // split-K partial sums (prefill scratch)
 #define GEMM_PART_SOFT ((size_t)1600000) // small calls' partial sums, floats (6.4 MB)
+// lfm_q6k_gemm, 6144 x 2048 by 8 / 300 / 1024 tokens: 29 / 60 / 180 us from the planes,
+// 148 / 160 / 240 with the copies; 16384 x 8192 by 2 / 300 / 1024: 64 / 450 / 1290 against
+// 923 / 1070 / 1300 (the two meet there).
+#define GEMM_DIRECT_TOKENS 1024u
+#define GEMM_DIRECT_PART ((uint64_t)500000) // its partial sums, floats (2 MB)
 #define GEMM_N64_BELOW 512u // two 128-token workgroups per CU on 256 CUs
 
 // Launches the matrix-core GEMM g (pair: gate + up + SwiGLU) over T tokens and nz
@@ -705,7 +710,7 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
     const bool exact = g.w.wide || (pair && g.w2.wide);
     // small ungrouped projections of up to 3072 rows (q/k/v, the out projections):
     // one 32-row tile per wave
-    const bool one_tile = small && !pair && (exact || (nz == 1 && g.zrows <= 3072));
+    const bool one_tile = small && !pair && (exact || g.w.planes || (nz == 1 && g.zrows <= 3072));
     // large single-weight calls whose 128-token grid would not give each CU two
     // workgroups (few row tiles: the 2048- and 3072-row projections) take 64 tokens
     // per workgroup
@@ -731,6 +736,7 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
             S = 1;
     }
     hipFunction_t f = small ? (pair ? (exact ? K->gemm_swiglu_t32x : K->gemm_swiglu_t32)
+                                    : g.w.planes ? K->gemm_q6_rows
                                     : one_tile ? (exact ? K->gemm_q6_t32x : K->gemm_q6_t32n1) : K->gemm_q6_t32)
                     : h16 ? (pair ? K->gemm_swiglu_h16 : n64 ? K->gemm_h16_n64 : K->gemm_h16)
                             : (pair ? (exact ? K->gemm_swiglu_x : K->gemm_swiglu)
@@ -785,69 +791,66 @@ extern "C" int lfm_q6k_gemm(const void *packed, uint64_t rows, uint64_t in_dim, 
     Kernels *K;
     RC(get_kernels(&K));
     hipStream_t s = (hipStream_t)stream;
+    // A call on a weight that is seen once does not pay for copies of it: up to
+    // GEMM_DIRECT_TOKENS tokens k_gemm_q6_rows reads the planes (small-call kernel:
+    // activations token-blocked, rows padded to 32), one wait and no device allocation of
+    // 2 MB or more for ordinary sizes (those take 35 us each to make and free).  Beyond,
+    // the large-call kernels over a tile copy and a binary16 copy.
+    const bool direct = T <= GEMM_DIRECT_TOKENS;
+    const size_t hrows = direct ? (T + 31) / 32 * 32 : T;
     uint16_t *hi = nullptr, *lo = nullptr;
-    float *scale = nullptr;
-    // small calls (T <= GEMM_TOKENS) use the token-blocked layout, rows padded to 32
-    const size_t hrows = T <= GEMM_TOKENS ? (T + 31) / 32 * 32 : T;
-    HIPCHK(hipMalloc(&hi, hrows * in_dim * 2));
-    HIPCHK(hipMalloc(&lo, hrows * in_dim * 2));
-    HIPCHK(hipMalloc(&scale, (size_t)T * 4));
-    float *bscale = nullptr; // small calls: the half-block scales of the blocked rows
-    if (T <= GEMM_TOKENS && hipMalloc(&bscale, hrows * (in_dim / 128) * 4) != hipSuccess) {
-        (void)hipFree(hi);
-        (void)hipFree(lo);
-        (void)hipFree(scale);
-        return fail(LFM_EDEVICE, "lfm_q6k_gemm: scale allocation failed");
-    }
+    float *scale = nullptr, *bscale = nullptr, *part = nullptr;
+    void *tiles = nullptr, *h16 = nullptr;
+    size_t part_cap = 0;
     SplitArgs sa;
     memset(&sa, 0, sizeof(sa));
-    sa.x = x;
-    sa.hi = hi;
-    sa.lo = lo;
-    sa.scale = scale;
-    sa.bscale = bscale;
-    sa.T = T;
-    sa.K = (uint32_t)in_dim;
-    sa.mode = T <= GEMM_TOKENS ? SPLIT_BLOCKED : SPLIT_ROWMAJOR;
-    int rc = launch(K->split_rows, dim3(T), 0, s, sa);
     GemmArgs ga;
     memset(&ga, 0, sizeof(ga));
-    void *tiles = nullptr, *h16 = nullptr;
-    if (rc == LFM_OK)
-        rc = make_tiles(K, s, q6view(packed, rows, in_dim), (uint32_t)rows, &tiles, &ga.w);
-    if (rc == LFM_OK && T > GEMM_TOKENS)
-        rc = make_h16(K, s, &ga.w, &h16);
-    ga.x_hi = hi;
-    ga.x_lo = lo;
-    ga.xscale = scale;
-    ga.bscale = bscale;
-    ga.ntok = T;
-    ga.zrows = (uint32_t)rows;
-    ga.c = y;
-    ga.ldc = (uint32_t)rows;
-    float *part = nullptr;
-    size_t part_cap = 0;
-    if (rc == LFM_OK && T <= GEMM_TOKENS) {
-        part_cap = std::min<size_t>(GEMM_PART_BYTES / 4, (size_t)T * rows * (in_dim / 256));
-        if (hipMalloc(&part, part_cap * 4) != hipSuccess)
-            rc = fail(LFM_EDEVICE, "lfm_q6k_gemm: scratch allocation failed");
-    }
-    uint64_t nd = 0;
-    if (rc == LFM_OK)
-        rc = launch_gemm(K, s, ga, false, T <= GEMM_TOKENS, T, 1, T, 0, part, part_cap, &nd);
-    if (rc == LFM_OK && hipStreamSynchronize(s) != hipSuccess)
+    auto run = [&]() -> int {
+        HIPCHK(hipMalloc(&hi, hrows * in_dim * 2));
+        HIPCHK(hipMalloc(&lo, hrows * in_dim * 2));
+        HIPCHK(hipMalloc(&scale, (size_t)T * 4));
+        if (direct) {
+            HIPCHK(hipMalloc(&bscale, hrows * (in_dim / 128) * 4));
+            const uint64_t slice = (uint64_t)T * rows;
+            if (in_dim > 256 && 2 * slice <= GEMM_DIRECT_PART) { // two K slices or more fit
+                part_cap = std::min<uint64_t>(GEMM_DIRECT_PART, slice * (in_dim / 256));
+                HIPCHK(hipMalloc(&part, part_cap * 4));
+            }
+        }
+        sa.x = x;
+        sa.hi = hi;
+        sa.lo = lo;
+        sa.scale = scale;
+        sa.bscale = bscale;
+        sa.T = T;
+        sa.K = (uint32_t)in_dim;
+        sa.mode = direct ? SPLIT_BLOCKED : SPLIT_ROWMAJOR;
+        RC(launch(K->split_rows, dim3(T), 0, s, sa));
+        if (direct) {
+            ga.w = Q6Tiles{(const uint8_t *)packed, 0, (uint32_t)(in_dim / 256), 0, (uint32_t)rows, 0, nullptr, 1};
+        } else {
+            RC(make_tiles(K, s, q6view(packed, rows, in_dim), (uint32_t)rows, &tiles, &ga.w));
+            RC(make_h16(K, s, &ga.w, &h16));
+        }
+        ga.x_hi = hi;
+        ga.x_lo = lo;
+        ga.xscale = scale;
+        ga.bscale = bscale;
+        ga.ntok = T;
+        ga.zrows = (uint32_t)rows;
+        ga.c = y;
+        ga.ldc = (uint32_t)rows;
+        uint64_t nd = 0;
+        return launch_gemm(K, s, ga, false, direct, T, 1, T, 0, part, part_cap, &nd);
+    };
+    int rc = run();
+    // also after a failure: nothing may still read the scratch
+    if (hipStreamSynchronize(s) != hipSuccess && rc == LFM_OK)
         rc = fail(LFM_EDEVICE, "lfm_q6k_gemm: synchronize failed");
-    (void)hipFree(hi);
-    (void)hipFree(lo);
-    (void)hipFree(scale);
-    if (bscale)
-        (void)hipFree(bscale);
-    if (part)
-        (void)hipFree(part);
-    if (tiles)
-        (void)hipFree(tiles);
-    if (h16)
-        (void)hipFree(h16);
+    for (void *p : {(void *)hi, (void *)lo, (void *)scale, (void *)bscale, (void *)part, tiles, h16})
+        if (p)
+            (void)hipFree(p);
     return rc;
 }
 

@@ -356,6 +356,7 @@ struct Q6Tiles {
                      // [-64, 64]: its weights sc (q - 32) can exceed 2048 in
                      // magnitude and need the GEMMs' two-part (_x) kernels
     const uint8_t *h16; // nullable: the binary16 fragment copy below (not wide only)
+    uint32_t planes; // 1: no tile copy, base is the Q6T planes of `rows` rows (k_gemm_q6_rows)
 };
 
 // The binary16 fragment copy of a Q6Tiles (the large-call GEMMs' A operands,

@@ -608,6 +608,25 @@ __device__ __forceinline__ void load_tile_chunks(const uint8_t *wb, size_t ntb, 
     A[1].sc = sc.y;
 }
 
+// The same chunks from the row-major planes of a Q6T of nblk blocks: half h of block
+// blk + ro, as they are (row_chunk_codes converts them).  blk is wave-uniform and ro
+// (the lane's row, in blocks) below 2^24, so an address is a scalar base and a 32-bit
+// offset.  Each load touches 32 rows' cache lines, which the next half block's loads
+// find in the vector cache.
+__device__ __forceinline__ void load_row_chunks(const uint8_t *wb, size_t nblk, size_t blk, uint32_t ro, uint32_t h,
+                                                uint32_t p, AChunk (&A)[2])
+{
+#pragma unroll
+    for (int ch = 0; ch < 2; ++ch) {
+        const uint8_t *pl = wb + blk * 128 + (4 * h + 2 * ch) * 16, *ph = wb + nblk * 128 + blk * 64 + (4 * h + 2 * ch) * 8;
+        A[ch].ql = *reinterpret_cast<const uint4 *>(pl + (ro * 128 + p * 16));
+        A[ch].qh = *reinterpret_cast<const uint2 *>(ph + (ro * 64 + p * 8));
+    }
+    const uint2 sc = *reinterpret_cast<const uint2 *>(wb + nblk * 192 + blk * 16 + h * 8 + ro * 16);
+    A[0].sc = sc.x;
+    A[1].sc = sc.y;
+}
+
 // binary16 bits of d of row r of tile-block tb
 __device__ __forceinline__ uint32_t tile_d(const uint8_t *wb, size_t ntb, size_t tb, uint32_t r)
 {
@@ -628,6 +647,17 @@ __device__ __forceinline__ void code_words(uint32_t A, uint32_t B, uint32_t H, u
     X[0] = (c0 << 2) | (c3 & M1);
     X[1] = (c1 << 2) | ((c3 >> 2) & M1);
     X[2] = (c2 << 2) | ((c3 >> 4) & M1);
+}
+
+// A chunk loaded by load_row_chunks -> the tile copy's form; dz: its block's d is zero.
+__device__ __forceinline__ void row_chunk_codes(AChunk &c, bool dz)
+{
+    uint32_t X0[3], X1[3];
+    code_words(c.ql.x, c.ql.z, c.qh.x, X0);
+    code_words(c.ql.y, c.ql.w, c.qh.y, X1);
+    c.ql = make_uint4(X0[0], X1[0], X0[1], X1[1]);
+    c.qh = make_uint2(X0[2], X1[2]);
+    c.sc = dz ? 0x80808080u : c.sc ^ 0x80808080u;
 }
 
 // Row-major Q6_K planes -> Q6Tiles (the layout is described with the struct).
@@ -752,6 +782,19 @@ __device__ __forceinline__ SplitFrag decode_frag_split(const AChunk &c, uint32_t
     }
     return {(half8){o[0][0], o[0][1], o[1][0], o[1][1], o[2][0], o[2][1], o[3][0], o[3][1]},
             (half8){r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]}};
+}
+
+// The r part alone, of weights w = decode_frag(c, s, ..).
+__device__ __forceinline__ half8 decode_frag_rest(const AChunk &c, uint32_t s, _Float16 scf, half8 w)
+{
+    const half2v sc2 = {scf, scf};
+    half2v r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const half2v q = codes256(code_bits(c, s, i >> 1), i & 1) - (half2v){(_Float16)288.0f, (_Float16)288.0f};
+        r[i] = __builtin_elementwise_fma(q, sc2, -(half2v){w[2 * i], w[2 * i + 1]});
+    }
+    return (half8){r[0][0], r[0][1], r[1][0], r[1][1], r[2][0], r[2][1], r[3][0], r[3][1]};
 }
 
 // Q6Tiles -> binary16 fragment copy (kargs.h TILE_H16): workgroup tb (one wave)
@@ -1419,10 +1462,14 @@ k_gemm_swiglu_h16(const GemmArgs a)
 // loads its next instructions use.  Same arithmetic per (row, token) as
 // gemm_body.  NI: 32-row tiles per wave (the pair form: its gate and up tile).
 // EXACT: weights in two parts as in gemm_body (the _x kernels).
-template <bool PAIR, int NI, int G, bool EXACT = false>
+// ROWS: the weights come from the row-major planes (Q6Tiles::planes) and each wave finds
+// out by itself whether a half block's scales need the two parts: a call on a weight it
+// sees once needs no tile copy and no flag from the device.
+template <bool PAIR, int NI, int G, bool EXACT = false, bool ROWS = false>
 __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
 {
     static_assert(!PAIR || NI == 2, "the pair form holds a gate and an up tile per wave");
+    static_assert(!ROWS || (!PAIR && !EXACT), "the row-major form takes one weight");
     constexpr uint32_t TMW = PAIR ? TM / 2 : 128 * NI; // rows of each weight per workgroup
     uint32_t z, mx, ny;
     {
@@ -1478,11 +1525,21 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
     constexpr uint32_t NBUF = G + 4;
     __shared__ __attribute__((aligned(16))) _Float16 Bs[NBUF][2 * 8 * 256];
     typedef AChunk BlockW[2][NI][2]; // a block's weights: [half][row tile][chunk]
+    // row-major: this lane's row of tile i (past the last one, that one: not stored),
+    // in blocks from the workgroup's first row
+    const size_t nblk = (size_t)a.w.rows * nb, blk0 = (size_t)m0 * nb + kb0;
+    uint32_t ro[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+        ro[i] = min(lb[i] + lr, a.zrows - 1 - m0) * nb;
     auto loadA = [=](uint32_t half, AChunk (&A)[NI][2]) {
         const uint32_t kb = kb0 + (half >> 1), h = half & 1;
 #pragma unroll
         for (int i = 0; i < NI; ++i)
-            load_tile_chunks<true>(PAIR && i ? a.w2.base : a.w.base, ntb, (size_t)wt[i] * nb + kb, h, lane, A[i]);
+            if constexpr (ROWS)
+                load_row_chunks(a.w.base, nblk, blk0 + (half >> 1), ro[i], h, p, A[i]);
+            else
+                load_tile_chunks<true>(PAIR && i ? a.w2.base : a.w.base, ntb, (size_t)wt[i] * nb + kb, h, lane, A[i]);
     };
     // stage st's tile into its buffer (this wave's two 16-byte pieces per lane)
     auto loadB = [&](uint32_t st) {
@@ -1497,7 +1554,8 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
     auto loadD = [=](uint32_t kb, uint32_t (&d)[NI], float (&ts)[2]) {
 #pragma unroll
         for (int i = 0; i < NI; ++i)
-            d[i] = tile_d(PAIR && i ? a.w2.base : a.w.base, ntb, (size_t)wt[i] * nb + kb0 + kb, lr);
+            d[i] = ROWS ? reinterpret_cast<const uint16_t *>(a.w.base + nblk * 208 + (blk0 + kb) * 2)[ro[i]]
+                        : tile_d(PAIR && i ? a.w2.base : a.w.base, ntb, (size_t)wt[i] * nb + kb0 + kb, lr);
         ts[0] = bsc[2 * (kb0 + kb)];
         ts[1] = bsc[2 * (kb0 + kb) + 1];
     };
@@ -1556,6 +1614,7 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
                 acc[i][e] *= c;
     };
     const uint32_t nst = nbl * 4;
+    bool two = false; // row-major: the current half block's weights are added in two parts
 
     // Stage s = 4 kb + j.  The workgroup meets at a barrier after every G-th stage
     // only: the first stage of a group issues the tiles of stages s + 4 .. s + 3 + G
@@ -1598,6 +1657,17 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
         half8 bch[4], bcl[4];
         // k-step kq reads k-piece 2 kq + p of row lr
         lds_frags_issue(lds_addr(Bs[st % NBUF]) + (p * 256 + lr * 8) * 2, bch, bcl);
+        if (ROWS && q == 0) {
+            uint32_t far = 0; // bit 7 of a byte: a scale outside [-64, 63]
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+#pragma unroll
+                for (int ch = 0; ch < 2; ++ch) {
+                    far |= A[i][ch].sc ^ (A[i][ch].sc << 1);
+                    row_chunk_codes(A[i][ch], dcur[i] == 0.f);
+                }
+            two = __ballot((far & 0x80808080u) != 0) != 0;
+        }
         if constexpr (!EXACT) {
         half8 afc[NI];
         // the stage's scales: sub-blocks 2q, 2q + 1 of each chunk
@@ -1625,6 +1695,13 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
 #pragma unroll
             for (int i = 0; i < NI; ++i)
                 acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i], bcl[kq], acc[i], 0, 0, 0);
+            if (ROWS && two) { // uniform
+#pragma unroll
+                for (int i = 0; i < NI; ++i)
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                        decode_frag_rest(A[i][kq & 1], 2 * q + (kq >> 1), ss[i][kq & 1].sc[(kq >> 1) & 1], afc[i]), bch[kq],
+                        acc[i], 0, 0, 0);
+            }
             if (kq < 3) {
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
@@ -1855,6 +1932,15 @@ extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_swiglu_t32(cons
 extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_t32n1(const GemmArgs a)
 {
     gemm_small_body<false, 1, 2>(a); // three workgroups per CU: 6 tile buffers fit their LDS
+}
+
+// Weights straight from the row-major planes (lfm_q6k_gemm): 168 VGPRs, three waves per
+// SIMD.  Converting a chunk to the tile copy's codes adds 26 operations to a half
+// block's 104 of decode; the tile copy alone took 7.6 us of kernel for 6144 x 2048 and
+// the waits, allocations and second copy around it 80 us.
+extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_gemm_q6_rows(const GemmArgs a)
+{
+    gemm_small_body<false, 1, 2, false, true>(a);
 }
 
 // Two-part weights (some |sc| > 64): one 32-row tile per wave for
