@@ -743,6 +743,14 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
                                     : n64 ? (exact ? K->gemm_q6_x : K->gemm_q6_n64) : K->gemm_q6);
     if (deferred)
         *deferred = S;
+    g.nz = nz;
+    if (g.counts && small) {
+        // the token tiles the lists can fill: each expert's last tile holds at least one
+        // of the T * n_used entries, and no list more than T
+        const uint64_t entries = (uint64_t)T * n_used;
+        grid.y = (uint32_t)std::min<uint64_t>({(uint64_t)grid.y * nz, entries, (entries + (uint64_t)nz * 31) / 32});
+        grid.z = 1;
+    }
     if (S == 1) {
         RC(launch_t(f, grid, GEMM_THREADS, 0, s, g));
         *dispatches += 1;
@@ -750,9 +758,8 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
     }
     g.part = part;
     g.ksplit = S;
-    g.nz = nz;
     g.part_rows = part_rows;
-    grid.z = nz * S;
+    grid.z = S; // (ungrouped: nz is 1; grouped: the tiles are in grid.y)
     RC(launch_t(f, grid, GEMM_THREADS, 0, s, g));
     if (deferred) {
         *dispatches += 1;

@@ -405,11 +405,11 @@ struct GemmArgs {
     uint32_t ntok, list_stride, zrows;
     float *c;
     uint32_t ldc, col0, mode;
-    // split over K (ksplit > 1): grid z = nz groups x ksplit slices; slice s covers
+    // split over K (ksplit > 1): grid z = ksplit slices; slice s covers
     // Q6_K blocks [s nb / ksplit, (s + 1) nb / ksplit) and writes its fp32 sums to
     // part[((s * (pair ? 2 : 1) + weight) * part_rows + out_row) * zrows + row]
     float *part;
-    uint32_t ksplit, nz, part_rows;
+    uint32_t ksplit, nz, part_rows; // nz: groups (experts, at most 64; one without lists)
     uint32_t rpz;           // small calls, grouped: blocked activation rows per group (x 32)
 };
 

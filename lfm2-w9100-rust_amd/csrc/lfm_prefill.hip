@@ -842,10 +842,9 @@ extern "C" __global__ __launch_bounds__(64) void k_q6_tile_h16(const TileH16Args
 //     sum_b d_b P_b / u with u the last nonzero d seen, so entering block b
 //     multiplies them by u / d_b (blocks with d = 0 contribute zero weights),
 //     and the epilogue multiplies by the final u.
-// Workgroup i runs on XCD i % 8; tiles are handed out so that each XCD takes a
-// contiguous run with the weight rows fastest, and the workgroups resident on
-// one XCD share activation tiles in its L2.  With ksplit > 1 the grid's z also
-// enumerates K slices: a workgroup runs its slice's blocks only and writes its
+// Tiles are handed out so that each XCD takes a contiguous run with the weight rows
+// fastest (GemmAt), and the workgroups resident on one XCD share activation tiles in
+// its L2.  With ksplit > 1 a workgroup runs its slice's blocks only and writes its
 // sums to part, which k_gemm_reduce adds up in slice order.
 // A lane's 16 accumulator rows of a 32-row tile are rb + 8 (e / 4) + e % 4 (rb =
 // the tile's first row + 4 p).  Writes v (add false) or adds it (add true) to those
@@ -880,6 +879,68 @@ __device__ __forceinline__ void store_rows16(float *out, uint32_t rb, uint32_t z
 // with whole-range scales at 7 / 64 / 512 / 1500 / 3000 tokens 596 / 588 / 1392 / 3165 /
 // 5266 us with four, 570 / 548 / 1286 / 2688 / 4440 us with three; error against 64-bit
 // arithmetic the same (the rest r xl is 2e-8 of a sum over uniform scales and codes).
+// Where workgroup i of a GEMM launch works.  It runs on XCD i % 8: work items are dealt
+// out in one contiguous run per XCD, row tiles mx fastest, then the token tiles ny, then
+// the groups z (experts), then K slices.
+struct GemmAt {
+    uint32_t z, mx, ny, ks, ntok;
+    bool ok;
+};
+__device__ __forceinline__ uint32_t xcd_item(uint32_t total, bool &ok)
+{
+    const uint32_t L = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const uint32_t q = total / 8, r = total % 8, xcd = L % 8, idx = L / 8;
+    ok = idx < q + (xcd < r ? 1u : 0u);
+    return xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
+}
+// Every group's possible tiles are items, those past its list's end empty.
+__device__ __forceinline__ GemmAt gemm_at(const GemmArgs &a)
+{
+    const uint32_t gx = gridDim.x, gy = gridDim.y;
+    GemmAt w;
+    uint32_t V = xcd_item(gx * gy * gridDim.z, w.ok);
+    w.mx = V % gx;
+    V /= gx;
+    w.ny = V % gy;
+    V /= gy;
+    w.z = a.counts ? V : 0u;
+    w.ks = a.counts ? 0u : V;
+    w.ntok = a.counts ? a.counts[w.z] : a.ntok;
+    return w;
+}
+// Grouped small calls: only the token tiles that the experts' lists fill are items (tiles
+// of ncol columns), counted here from the lists' lengths by every wave, so that the XCDs'
+// shares are equal whatever the routing; the launch has workgroups for the most tiles a
+// routing can need, and the others end here.  With every possible tile an item each XCD
+// had four experts: for 7 tokens, with about 19 experts in use, the busiest XCD had 1.7 -
+// 1.9 times the mean, and the gate/up pair took 53 us instead of 45 (203 tokens: 73 instead of
+// 60).  Large calls keep the experts whole: their lists differ by 5 % from XCD to XCD and
+// 3840 tokens of the model took 28.7 ms dealt out like this, 28.0 ms as they are.
+__device__ __forceinline__ GemmAt gemm_at_group(const GemmArgs &a, uint32_t gx, uint32_t ncol)
+{
+    const uint32_t lane = threadIdx.x & 63, c = lane < a.nz ? a.counts[lane] : 0u;
+    // inclusive sums of the experts' tile counts
+    int t = (int)((c + ncol - 1) / ncol);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x111, 0xf, 0xf, false); // row_shr 1, 2, 4, 8
+    t += __builtin_amdgcn_update_dpp(0, t, 0x112, 0xf, 0xf, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x114, 0xf, 0xf, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x118, 0xf, 0xf, false);
+    t += __builtin_amdgcn_update_dpp(0, t, 0x142, 0xa, 0xf, false); // row_bcast 15, 31
+    t += __builtin_amdgcn_update_dpp(0, t, 0x143, 0xc, 0xf, false);
+    const uint32_t per = (uint32_t)__builtin_amdgcn_readlane(t, 63) * gx;
+    GemmAt w;
+    const uint32_t V = xcd_item(per * max(a.ksplit, 1u), w.ok);
+    if (!w.ok)
+        return w;
+    w.ks = V / per;
+    const uint32_t i = V - w.ks * per, tile = i / gx;
+    w.mx = i - tile * gx;
+    w.z = (uint32_t)__popcll(__ballot((uint32_t)t <= tile));
+    w.ny = tile - (w.z ? (uint32_t)__builtin_amdgcn_readlane(t, w.z - 1) : 0u);
+    w.ntok = (uint32_t)__builtin_amdgcn_readlane((int)c, w.z);
+    return w;
+}
+
 template <bool PAIR, int NJ, bool EXACT = false>
 __device__ __forceinline__ void gemm_body(const GemmArgs &a)
 {
@@ -887,25 +948,16 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
     // rows of each weight per workgroup; the workgroup's 256 "tile rows" v are
     // rows m0 + v (single) or rows m0 + (v & 127) of weight v >> 7 (pair)
     constexpr uint32_t TMW = PAIR ? TM / 2 : TM;
-    uint32_t z, mx, ny;
-    {
-        const uint32_t gx = gridDim.x, gy = gridDim.y, total = gx * gy * gridDim.z;
-        const uint32_t L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-        const uint32_t q = total / 8, r = total % 8, xcd = L % 8, idx = L / 8;
-        const uint32_t V = xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
-        mx = V % gx;
-        ny = (V / gx) % gy;
-        z = V / (gx * gy);
-    }
+    const GemmAt at = gemm_at(a);
+    if (!at.ok)
+        return;
+    const uint32_t z = at.z, mx = at.mx, ny = at.ny, ks = at.ks;
     // K slice of this workgroup (the whole row unless split)
     const uint32_t nb = a.w.nb, K = nb * 256;
-    const uint32_t ks = a.ksplit > 1 ? z / a.nz : 0;
-    if (a.ksplit > 1)
-        z -= ks * a.nz;
     const uint32_t kb0 = a.ksplit > 1 ? ks * nb / a.ksplit : 0;
     const uint32_t nbl = a.ksplit > 1 ? (ks + 1) * nb / a.ksplit - kb0 : nb;
     const uint32_t m0 = mx * TMW, n0 = ny * TNW;
-    const uint32_t ntok = a.counts ? a.counts[z] : a.ntok;
+    const uint32_t ntok = at.ntok;
     if (m0 >= a.zrows || n0 >= ntok)
         return;
     const uint32_t *tokl = a.tok ? a.tok + (size_t)z * a.list_stride : nullptr;
@@ -1238,26 +1290,24 @@ __device__ __forceinline__ void gemm_body_h(const GemmArgs &a)
 {
     constexpr uint32_t TNW = 32 * NJ;
     constexpr uint32_t TMW = PAIR ? TM / 2 : TM;
-    uint32_t z, mx, ny;
-    {
-        const uint32_t gx = gridDim.x, gy = gridDim.y, total = gx * gy * gridDim.z;
-        const uint32_t L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-        const uint32_t q = total / 8, r = total % 8, xcd = L % 8, idx = L / 8;
-        const uint32_t V = xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
-        // Within a weight slice, groups of 8 token tiles with the row tiles next: the
-        // workgroups resident on one XCD (a run of consecutive V) then cover about 8
-        // row tiles x 8 token tiles, whose weights and activations its L2 shares.
+    GemmAt at = gemm_at(a);
+    if (!at.ok)
+        return;
+    if (!a.counts && gridDim.x > 8) {
+        // Groups of 8 token tiles with the row tiles next: the workgroups resident on one
+        // XCD (a run of consecutive V) then cover about 8 row tiles x 8 token tiles, whose
+        // weights and activations its L2 shares.
         // (Row tiles fastest over all token tiles, as gemm_body orders them, reads
         // the whole weight once per token tile: 2.4 times the Q6_K bytes here.)
-        const uint32_t per = gx * gy, Vz = V % per, g = Vz / (gx * 8), w = Vz - g * gx * 8;
-        const uint32_t ng = min(8u, gy - g * 8);
-        mx = gx > 8 ? w / ng : Vz % gx;
-        ny = gx > 8 ? g * 8 + w % ng : Vz / gx;
-        z = V / per;
+        const uint32_t gx = gridDim.x, V = at.ny * gx + at.mx, g = V / (gx * 8), w = V - g * gx * 8;
+        const uint32_t ng = min(8u, gridDim.y - g * 8);
+        at.mx = w / ng;
+        at.ny = g * 8 + w % ng;
     }
+    const uint32_t z = at.z, mx = at.mx, ny = at.ny;
     const uint32_t nb = a.w.nb, K = nb * 256;
     const uint32_t m0 = mx * TMW, n0 = ny * TNW;
-    const uint32_t ntok = a.counts ? a.counts[z] : a.ntok;
+    const uint32_t ntok = at.ntok;
     if (m0 >= a.zrows || n0 >= ntok)
         return;
     const uint32_t *tokl = a.tok ? a.tok + (size_t)z * a.list_stride : nullptr;
@@ -1471,24 +1521,15 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
     static_assert(!PAIR || NI == 2, "the pair form holds a gate and an up tile per wave");
     static_assert(!ROWS || (!PAIR && !EXACT), "the row-major form takes one weight");
     constexpr uint32_t TMW = PAIR ? TM / 2 : 128 * NI; // rows of each weight per workgroup
-    uint32_t z, mx, ny;
-    {
-        const uint32_t gx = gridDim.x, gy = gridDim.y, total = gx * gy * gridDim.z;
-        const uint32_t L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-        const uint32_t q = total / 8, r = total % 8, xcd = L % 8, idx = L / 8;
-        const uint32_t V = xcd < r ? xcd * (q + 1) + idx : r * (q + 1) + (xcd - r) * q + idx;
-        mx = V % gx;
-        ny = (V / gx) % gy;
-        z = V / (gx * gy);
-    }
+    const GemmAt at = a.counts ? gemm_at_group(a, (a.zrows + TMW - 1) / TMW, 32) : gemm_at(a);
+    if (!at.ok)
+        return;
+    const uint32_t z = at.z, mx = at.mx, ny = at.ny, ks = at.ks;
     const uint32_t nb = a.w.nb, K = nb * 256;
-    const uint32_t ks = a.ksplit > 1 ? z / a.nz : 0;
-    if (a.ksplit > 1)
-        z -= ks * a.nz;
     const uint32_t kb0 = a.ksplit > 1 ? ks * nb / a.ksplit : 0;
     const uint32_t nbl = a.ksplit > 1 ? (ks + 1) * nb / a.ksplit - kb0 : nb;
     const uint32_t m0 = mx * TMW, n0 = ny * 32;
-    const uint32_t ntok = a.counts ? a.counts[z] : a.ntok;
+    const uint32_t ntok = at.ntok;
     if (m0 >= a.zrows || n0 >= ntok)
         return;
     const uint32_t *tokl = a.tok ? a.tok + (size_t)z * a.list_stride : nullptr;

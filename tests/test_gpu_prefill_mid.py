@@ -86,3 +86,24 @@ def test_real_width_whole_equals_chunks(real, n):
     lc, sc = e.snapshot_resident_logits(), state(e, n)
     assert rel_l2(lw, lc) <= 2e-5
     check_same(hp, n, sw, sc)
+
+
+@pytest.mark.parametrize("n", [2, 33, 200, 750])
+@pytest.mark.parametrize("sigma", [0.0, 4.0])
+def test_expert_lists_of_any_length(gpu, oracle, n, sigma):
+    """64 experts top-4: a spread of 4 in the selection bias sends every token to the
+    same few experts (lists of n tokens beside empty ones), 0 spreads them; either way
+    every list's tiles are found, on both sides of the line between the call sizes."""
+    hp = gpu.make_hparams(dim=512, heads=8, n_layers=4, attention_layers=(1,), kv=2, vocab=1000,
+                          eos=1 << 30, n_expert=64, n_used=4, expert_ff=256, n_ff=512, dense_lead=1)
+    tensors = model_tensors(hp, gpu.synth_opts(0x2545F4914F6CDD1D, bias_sigma=sigma))
+    prompt = ids(n, hp.vocab, n)
+    g = gpu_engine(hp, tensors, ctx=768)
+    o = oracle_engine(oracle, hp, tensors, ctx=768)
+    g.set_route_log(True)
+    lg, lo = g.forward(prompt, 0), o.forward(prompt, 0)
+    counts = np.bincount(g.prefill_routes(1)[1].reshape(-1), minlength=64)
+    assert counts.sum() == 4 * n and (sigma == 0.0 or counts.max() == n)
+    assert rel_l2(lg, lo) <= 1e-3
+    assert rel_l2(state(g, n), np.frombuffer(o.snapshot(n), np.float32)) <= 1e-3
+    g.close()
