@@ -828,7 +828,7 @@ extern "C" __global__ __launch_bounds__(64) void k_q6_tile_h16(const TileH16Args
 // multiplies the gate weight w and the up weight w2 by the same activations and
 // writes silu(gate) * up (lfm.rs:578-582 SwiGLU, g / (1 + e^-g) * u).
 //
-// A workgroup computes 256 weight rows x 128 tokens: wave w owns rows 64w..64w+63
+// A workgroup computes 256 weight rows x 128 tokens (32 NJ): wave w owns rows 64w..64w+63
 // for all 128 tokens (2 x 4 tiles of v_mfma_f32_32x32x16_f16, hi and lo
 // activation halves); in the pair form its two row tiles are the same 32 rows of
 // the gate and of the up weight (128 rows of each per workgroup), so a lane holds
@@ -879,6 +879,12 @@ __device__ __forceinline__ void store_rows16(float *out, uint32_t rb, uint32_t z
 // with whole-range scales at 7 / 64 / 512 / 1500 / 3000 tokens 596 / 588 / 1392 / 3165 /
 // 5266 us with four, 570 / 548 / 1286 / 2688 / 4440 us with three; error against 64-bit
 // arithmetic the same (the rest r xl is 2e-8 of a sum over uniform scales and codes).
+// The activation tiles (hi, lo, two buffers) and row factors of a large-call workgroup.
+struct LdsTiles {
+    _Float16 *h0, *h1, *l0, *l1;
+    float (*rsh)[2][TM];
+};
+
 // Where workgroup i of a GEMM launch works.  It runs on XCD i % 8: work items are dealt
 // out in one contiguous run per XCD, row tiles mx fastest, then the token tiles ny, then
 // the groups z (experts), then K slices.
@@ -941,25 +947,21 @@ __device__ __forceinline__ GemmAt gemm_at_group(const GemmArgs &a, uint32_t gx, 
     return w;
 }
 
-template <bool PAIR, int NJ, bool EXACT = false>
-__device__ __forceinline__ void gemm_body(const GemmArgs &a)
+// NJ: 32-column token tiles that the workgroup computes, from column n0 (a kernel of
+// TNW-column workgroups runs the form that its last columns fill, gemm_tiles).
+template <bool PAIR, int NJ, bool EXACT>
+__device__ __forceinline__ void gemm_body(const GemmArgs &a, const GemmAt &at, uint32_t n0, const LdsTiles &S)
 {
-    constexpr uint32_t TNW = 32 * NJ; // token columns per workgroup (128, or 32 for small calls)
     // rows of each weight per workgroup; the workgroup's 256 "tile rows" v are
     // rows m0 + v (single) or rows m0 + (v & 127) of weight v >> 7 (pair)
     constexpr uint32_t TMW = PAIR ? TM / 2 : TM;
-    const GemmAt at = gemm_at(a);
-    if (!at.ok)
-        return;
-    const uint32_t z = at.z, mx = at.mx, ny = at.ny, ks = at.ks;
+    const uint32_t z = at.z, ks = at.ks;
     // K slice of this workgroup (the whole row unless split)
     const uint32_t nb = a.w.nb, K = nb * 256;
     const uint32_t kb0 = a.ksplit > 1 ? ks * nb / a.ksplit : 0;
     const uint32_t nbl = a.ksplit > 1 ? (ks + 1) * nb / a.ksplit - kb0 : nb;
-    const uint32_t m0 = mx * TMW, n0 = ny * TNW;
+    const uint32_t m0 = at.mx * TMW;
     const uint32_t ntok = at.ntok;
-    if (m0 >= a.zrows || n0 >= ntok)
-        return;
     const uint32_t *tokl = a.tok ? a.tok + (size_t)z * a.list_stride : nullptr;
     const uint32_t *slotl = a.slot ? a.slot + (size_t)z * a.list_stride : nullptr;
     const __amdgpu_buffer_rsrc_t xh = act_rsrc(a.x_hi), xl = act_rsrc(a.x_lo);
@@ -967,9 +969,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
     // (unrolled) stage parity: the compiler can then tell that a stage's LDS reads do
     // not touch the buffer the next tile is being loaded into, and does not wait for
     // that load before them
-    __shared__ __attribute__((aligned(16))) _Float16 Bh0[TNW * TK], Bh1[TNW * TK];
-    __shared__ __attribute__((aligned(16))) _Float16 Bl0[TNW * TK], Bl1[TNW * TK];
-    __shared__ float dsh[2][TM], rsh[2][TM];
+    _Float16 *const Bh0 = S.h0, *const Bh1 = S.h1, *const Bl0 = S.l0, *const Bl1 = S.l1;
+    float(&rsh)[2][TM] = *S.rsh;
     // the wave index as a wave-uniform value, so that the row-tile and weight
     // addresses derived from it stay in scalar registers
     const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -1037,7 +1038,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
     // thread tid keeps tile row tid's running scale u (TM == GEMM_NTH)
     float u = 1.0f;
     auto set_d = [&](uint32_t slot, float d) {
-        dsh[slot][tid] = d;
         const bool nz = d != 0.f;
         rsh[slot][tid] = nz ? u / d : 1.0f;
         u = nz ? d : u;
@@ -1099,7 +1099,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i], bfh[j & 1], acc[i][j], 0, 0, 0);
-                if (j == 1 && ks < 3) {
+                if (j == (NJ > 1 ? 1 : 0) && ks < 3) {
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
                         afn[i] = decode_frag(A[i][(ks + 1) & 1], 2 * q + ((ks + 1) >> 1), ss[i][(ks + 1) & 1]);
@@ -1144,7 +1144,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].r, bfh[j & 1], acc[i][j], 0, 0, 0);
-                if (j == 1 && ks < 3) {
+                if (j == (NJ > 1 ? 1 : 0) && ks < 3) {
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
                         afn[i] = decode_frag_split(A[i][(ks + 1) & 1], 2 * q + ((ks + 1) >> 1),
@@ -1244,40 +1244,6 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a)
     }
 }
 
-extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-k_gemm_q6(const GemmArgs a)
-{
-    gemm_body<false, 4>(a);
-}
-
-// 64 token columns per workgroup: for projections whose 128-column grid would leave
-// CUs without a second workgroup (few row tiles)
-extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-k_gemm_q6_n64(const GemmArgs a)
-{
-    gemm_body<false, 2>(a);
-}
-
-extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-k_gemm_q6_swiglu(const GemmArgs a)
-{
-    gemm_body<true, 4>(a);
-}
-
-// Two-part weights (some |sc| > 64): 64 token columns per workgroup, so that the second
-// set of weight fragments fits the registers.
-extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-k_gemm_q6_x(const GemmArgs a)
-{
-    gemm_body<false, 2, true>(a);
-}
-
-extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-k_gemm_q6_swiglu_x(const GemmArgs a)
-{
-    gemm_body<true, 2, true>(a);
-}
-
 // The large-call GEMM over the binary16 fragment copy (Q6Tiles::h16, made once at
 // finalize by k_q6_tile_h16): gemm_body's workgroup tiles, activation staging,
 // block-scale folding and epilogue, but each wave loads its A fragments ready-made,
@@ -1286,36 +1252,17 @@ k_gemm_q6_swiglu_x(const GemmArgs a)
 // fragment reads and MFMAs.  The products are those of gemm_body (the
 // copy holds the fragments its decode forms).  Large calls only: one K slice.
 template <bool PAIR, int NJ>
-__device__ __forceinline__ void gemm_body_h(const GemmArgs &a)
+__device__ __forceinline__ void gemm_body_h(const GemmArgs &a, const GemmAt &at, uint32_t n0, const LdsTiles &S)
 {
-    constexpr uint32_t TNW = 32 * NJ;
     constexpr uint32_t TMW = PAIR ? TM / 2 : TM;
-    GemmAt at = gemm_at(a);
-    if (!at.ok)
-        return;
-    if (!a.counts && gridDim.x > 8) {
-        // Groups of 8 token tiles with the row tiles next: the workgroups resident on one
-        // XCD (a run of consecutive V) then cover about 8 row tiles x 8 token tiles, whose
-        // weights and activations its L2 shares.
-        // (Row tiles fastest over all token tiles, as gemm_body orders them, reads
-        // the whole weight once per token tile: 2.4 times the Q6_K bytes here.)
-        const uint32_t gx = gridDim.x, V = at.ny * gx + at.mx, g = V / (gx * 8), w = V - g * gx * 8;
-        const uint32_t ng = min(8u, gridDim.y - g * 8);
-        at.mx = w / ng;
-        at.ny = g * 8 + w % ng;
-    }
-    const uint32_t z = at.z, mx = at.mx, ny = at.ny;
-    const uint32_t nb = a.w.nb, K = nb * 256;
-    const uint32_t m0 = mx * TMW, n0 = ny * TNW;
+    const uint32_t z = at.z, nb = a.w.nb, K = nb * 256;
+    const uint32_t m0 = at.mx * TMW;
     const uint32_t ntok = at.ntok;
-    if (m0 >= a.zrows || n0 >= ntok)
-        return;
     const uint32_t *tokl = a.tok ? a.tok + (size_t)z * a.list_stride : nullptr;
     const uint32_t *slotl = a.slot ? a.slot + (size_t)z * a.list_stride : nullptr;
     const __amdgpu_buffer_rsrc_t xh = act_rsrc(a.x_hi), xl = act_rsrc(a.x_lo);
-    __shared__ __attribute__((aligned(16))) _Float16 Bh0[TNW * TK], Bh1[TNW * TK];
-    __shared__ __attribute__((aligned(16))) _Float16 Bl0[TNW * TK], Bl1[TNW * TK];
-    __shared__ float dsh[2][TM], rsh[2][TM];
+    _Float16 *const Bh0 = S.h0, *const Bh1 = S.h1, *const Bl0 = S.l0, *const Bl1 = S.l1;
+    float(&rsh)[2][TM] = *S.rsh;
     const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const uint32_t p = lane >> 5, lr = lane & 31;
     const size_t ntb = (size_t)a.w.tiles * nb;
@@ -1367,7 +1314,6 @@ __device__ __forceinline__ void gemm_body_h(const GemmArgs &a)
     };
     float u = 1.0f;
     auto set_d = [&](uint32_t slot, float d) {
-        dsh[slot][tid] = d;
         const bool nz = d != 0.f;
         rsh[slot][tid] = nz ? u / d : 1.0f;
         u = nz ? d : u;
@@ -1483,23 +1429,114 @@ __device__ __forceinline__ void gemm_body_h(const GemmArgs &a)
     }
 }
 
+// A large-call kernel of 32 * NJ token columns per workgroup: the body for as many
+// 32-column tiles as hold tokens (an expert's last tile, a call's last columns).  At 3840
+// tokens an expert has 480 of them, and 128-column tiles alone multiply 10 % of padding
+// (64-column ones at 1500 tokens 16 %), 32-column ends 3 and 8 %: 3840 tokens of the model
+// 27.5 -> 26.8 ms, a 4-layer block of wide scales at 1500 tokens 2262 -> 2226 us.
+template <int N> struct Tiles {
+    static constexpr int n = N;
+};
+template <bool PAIR, int NJ, bool EXACT, bool H16>
+__device__ __forceinline__ void gemm_tiles(const GemmArgs &a)
+{
+    constexpr uint32_t TNW = 32 * NJ, TMW = PAIR ? TM / 2 : TM;
+    __shared__ __attribute__((aligned(16))) _Float16 Bh0[TNW * TK], Bh1[TNW * TK];
+    __shared__ __attribute__((aligned(16))) _Float16 Bl0[TNW * TK], Bl1[TNW * TK];
+    __shared__ float rsh[2][TM];
+    GemmAt at = gemm_at(a);
+    if (!at.ok)
+        return;
+    if (H16 && !a.counts && gridDim.x > 8) {
+        // Groups of 8 token tiles with the row tiles next: the workgroups resident on one
+        // XCD (a run of consecutive V) then cover about 8 row tiles x 8 token tiles, whose
+        // weights and activations its L2 shares.
+        // (Row tiles fastest over all token tiles, as gemm_body orders them, reads
+        // the whole weight once per token tile: 2.4 times the Q6_K bytes here.)
+        const uint32_t gx = gridDim.x, V = at.ny * gx + at.mx, g = V / (gx * 8), w = V - g * gx * 8;
+        const uint32_t ng = min(8u, gridDim.y - g * 8);
+        at.mx = w / ng;
+        at.ny = g * 8 + w % ng;
+    }
+    const uint32_t n0 = at.ny * TNW;
+    if (at.mx * TMW >= a.zrows || n0 >= at.ntok)
+        return;
+    const LdsTiles S{Bh0, Bh1, Bl0, Bl1, &rsh};
+    auto run = [&](auto nj) {
+        if constexpr (H16)
+            gemm_body_h<PAIR, decltype(nj)::n>(a, at, n0, S);
+        else
+            gemm_body<PAIR, decltype(nj)::n, EXACT>(a, at, n0, S);
+    };
+    const uint32_t left = at.ntok - n0;
+    if constexpr (NJ == 4) {
+        if (left > 96)
+            run(Tiles<4>());
+        else if (left > 64)
+            run(Tiles<3>());
+        else if (left > 32)
+            run(Tiles<2>());
+        else
+            run(Tiles<1>());
+    } else {
+        if (left > 32)
+            run(Tiles<2>());
+        else
+            run(Tiles<1>());
+    }
+}
+
+extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_gemm_q6(const GemmArgs a)
+{
+    gemm_tiles<false, 4, false, false>(a);
+}
+
+// 64 token columns per workgroup: for projections whose 128-column grid would leave
+// CUs without a second workgroup (few row tiles)
+extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_gemm_q6_n64(const GemmArgs a)
+{
+    gemm_tiles<false, 2, false, false>(a);
+}
+
+extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_gemm_q6_swiglu(const GemmArgs a)
+{
+    gemm_tiles<true, 4, false, false>(a);
+}
+
+// Two-part weights (some |sc| > 64): 64 token columns per workgroup, so that the second
+// set of weight fragments fits the registers.
+extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_gemm_q6_x(const GemmArgs a)
+{
+    gemm_tiles<false, 2, true, false>(a);
+}
+
+extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+k_gemm_q6_swiglu_x(const GemmArgs a)
+{
+    gemm_tiles<true, 2, true, false>(a);
+}
+
 extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 k_gemm_h16(const GemmArgs a)
 {
-    gemm_body_h<false, 4>(a);
+    gemm_tiles<false, 4, false, true>(a);
 }
 
 // (152 VGPRs: three waves per SIMD)
 extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(3, 3))) void
 k_gemm_h16_n64(const GemmArgs a)
 {
-    gemm_body_h<false, 2>(a);
+    gemm_tiles<false, 2, false, true>(a);
 }
 
 extern "C" __global__ __launch_bounds__(GEMM_NTH) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 k_gemm_swiglu_h16(const GemmArgs a)
 {
-    gemm_body_h<true, 4>(a);
+    gemm_tiles<true, 4, false, true>(a);
 }
 
 // The same products for calls of up to 128 tokens (chunked prefill: about 8

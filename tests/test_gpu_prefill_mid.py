@@ -107,3 +107,23 @@ def test_expert_lists_of_any_length(gpu, oracle, n, sigma):
     assert rel_l2(lg, lo) <= 1e-3
     assert rel_l2(state(g, n), np.frombuffer(o.snapshot(n), np.float32)) <= 1e-3
     g.close()
+
+
+@pytest.mark.parametrize("full_scales,h16", [(0, "1"), (0, "0"), (1, "1")])
+@pytest.mark.parametrize("n", [129, 160, 161, 193, 225, 256])
+def test_last_columns_of_large_calls(gpu, oracle, monkeypatch, n, full_scales, h16):
+    """Large-call kernels (a model narrower than 512 runs them from 129 tokens) with 1, 32,
+    33, 65, 97 and 128 columns in the last 128-token tile: each form of the last tile, and
+    the experts' own list ends, for the binary16 copies, the Q6_K weights and the two-part
+    weights."""
+    monkeypatch.setenv("LFM_PREFILL_H16", h16)
+    hp = gpu.make_hparams(dim=256, heads=4, n_layers=4, attention_layers=(1,), kv=2, vocab=1000,
+                          eos=1 << 30, n_expert=8, n_used=4, expert_ff=256, n_ff=512, dense_lead=1)
+    tensors = model_tensors(hp, gpu.synth_opts(0x9E3779B97F4A7C15, bias_sigma=0.1, full_scales=full_scales))
+    prompt = ids(n, hp.vocab, n)
+    g = gpu_engine(hp, tensors, ctx=256)
+    o = oracle_engine(oracle, hp, tensors, ctx=256)
+    lg, lo = g.forward(prompt, 0), o.forward(prompt, 0)
+    assert rel_l2(lg, lo) <= 1e-3
+    assert rel_l2(state(g, n), np.frombuffer(o.snapshot(n), np.float32)) <= 1e-3
+    g.close()
