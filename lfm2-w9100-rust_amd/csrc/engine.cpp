@@ -110,7 +110,7 @@ struct Shape {
 struct Kernels {
     hipModule_t mod = nullptr, pmod = nullptr;
     hipFunction_t split_rows, split_rows_ext, gemm_q6, conv_prefill, rope_kv_prefill, attn_prefill,
-        gemm_swiglu, gemm_q6_t32, gemm_q6_t32n1, gemm_swiglu_t32, gemm_reduce, attn_merge_split, router_small, router_mfma, router_split, route_topk, route_group, combine_prefill, embed_rows,
+        gemm_swiglu, gemm_q6_t32n1, gemm_swiglu_t32, gemm_reduce, attn_merge_split, router_small, router_mfma, router_split, route_topk, route_group, combine_prefill, embed_rows,
         tile_pack, gemm_q6_n64, gemm_q6_x, gemm_swiglu_x, gemm_q6_t32x, gemm_swiglu_t32x, tile_h16, gemm_h16, gemm_q6_rows,
         gemm_h16_n64, gemm_swiglu_h16;
     hipFunction_t matvec_long, attn, attn_merge, router, moe_down, argmax, argmax_final, advance,
@@ -245,7 +245,7 @@ static int get_kernels(Kernels **out)
                 {&k->gemm_swiglu, "k_gemm_q6_swiglu"}, {&k->router_mfma, "k_router_mfma"}, {&k->router_split, "k_router_split"},
                 {&k->route_topk, "k_route_topk"},       {&k->route_group, "k_route_group"},
                 {&k->combine_prefill, "k_combine_prefill"}, {&k->gemm_reduce, "k_gemm_reduce"},
-                {&k->gemm_q6_t32, "k_gemm_q6_t32"},     {&k->gemm_swiglu_t32, "k_gemm_q6_swiglu_t32"},
+                {&k->gemm_swiglu_t32, "k_gemm_q6_swiglu_t32"},
                 {&k->gemm_q6_t32n1, "k_gemm_q6_t32n1"},
                 {&k->attn_merge_split, "k_attn_merge_split"}, {&k->router_small, "k_router_prefill_small"},
                 {&k->embed_rows, "k_embed_rows"}, {&k->tile_pack, "k_q6_tile_pack"},
@@ -708,9 +708,10 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
     // weights with scales outside [-64, 64] take the two-part kernels (one 32-row
     // tile per wave for small single-weight calls, 64 tokens per large workgroup)
     const bool exact = g.w.wide || (pair && g.w2.wide);
-    // small ungrouped projections of up to 3072 rows (q/k/v, the out projections):
-    // one 32-row tile per wave
-    const bool one_tile = small && !pair && (exact || g.w.planes || (nz == 1 && g.zrows <= 3072));
+    // small single-weight calls: one 32-row tile per wave.  (Two tiles, for 6144-row
+    // and expert weights, left CUs idle: a 4-layer block at 7 / 37 / 203 / 512 tokens from 700 took
+    // 359 / 400 / 577 / 971 us with them, 345 / 391 / 553 / 934 without.)
+    const bool one_tile = small && !pair;
     // large single-weight calls whose 128-token grid would not give each CU two
     // workgroups (few row tiles: the 2048- and 3072-row projections) take 64 tokens
     // per workgroup
@@ -721,9 +722,16 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
     const bool h16 = !small && !exact && g.w.h16 && (!pair || g.w2.h16);
     dim3 grid = gemm_grid(g.zrows, T, nz, pair || one_tile ? GEMM_ROWS / 2 : GEMM_ROWS,
                           small ? 32 : t64 ? GEMM_TOKENS / 2 : GEMM_TOKENS);
+    if (g.counts && small) {
+        // the token tiles the lists can fill: each expert's last tile holds at least one
+        // of the T * n_used entries, and no list more than T
+        const uint64_t entries = (uint64_t)T * n_used;
+        grid.y = (uint32_t)std::min<uint64_t>({(uint64_t)grid.y * nz, entries, (entries + (uint64_t)nz * 31) / 32});
+        grid.z = 1;
+    }
     uint32_t S = 1;
     if (part && small) {
-        const uint32_t wgs = grid.x * grid.y * grid.z;
+        const uint32_t wgs = grid.x * grid.y;
         const size_t per = (size_t)(pair ? 2 : 1) * part_rows * g.zrows;
         S = std::min<uint32_t>(std::max<uint32_t>(1, 1024 / wgs), g.w.nb);
         // and at most GEMM_PART_SOFT floats of partial sums: past that, writing and
@@ -737,20 +745,13 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
     }
     hipFunction_t f = small ? (pair ? (exact ? K->gemm_swiglu_t32x : K->gemm_swiglu_t32)
                                     : g.w.planes ? K->gemm_q6_rows
-                                    : one_tile ? (exact ? K->gemm_q6_t32x : K->gemm_q6_t32n1) : K->gemm_q6_t32)
+                                    : exact ? K->gemm_q6_t32x : K->gemm_q6_t32n1)
                     : h16 ? (pair ? K->gemm_swiglu_h16 : n64 ? K->gemm_h16_n64 : K->gemm_h16)
                             : (pair ? (exact ? K->gemm_swiglu_x : K->gemm_swiglu)
                                     : n64 ? (exact ? K->gemm_q6_x : K->gemm_q6_n64) : K->gemm_q6);
     if (deferred)
         *deferred = S;
     g.nz = nz;
-    if (g.counts && small) {
-        // the token tiles the lists can fill: each expert's last tile holds at least one
-        // of the T * n_used entries, and no list more than T
-        const uint64_t entries = (uint64_t)T * n_used;
-        grid.y = (uint32_t)std::min<uint64_t>({(uint64_t)grid.y * nz, entries, (entries + (uint64_t)nz * 31) / 32});
-        grid.z = 1;
-    }
     if (S == 1) {
         RC(launch_t(f, grid, GEMM_THREADS, 0, s, g));
         *dispatches += 1;

@@ -1993,20 +1993,13 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
     }
 }
 
-// Two 32-row tiles per wave (two workgroups per CU): a barrier once per block.
-extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_t32(const GemmArgs a)
-{
-    gemm_small_body<false, 2, 4>(a);
-}
-
+// A gate and an up tile per wave (two workgroups per CU): a barrier once per block.
 extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_swiglu_t32(const GemmArgs a)
 {
     gemm_small_body<true, 2, 4>(a);
 }
 
-// One 32-row tile per wave (128 rows per workgroup, 144 VGPRs: three waves per
-// SIMD): faster for the ungrouped projections of up to 2048 rows at 64 tokens,
-// slower for the expert and 6144-row shapes.
+// One 32-row tile per wave (128 rows per workgroup, 140 VGPRs: three waves per SIMD).
 extern "C" __global__ __launch_bounds__(GEMM_NTH) void k_gemm_q6_t32n1(const GemmArgs a)
 {
     gemm_small_body<false, 1, 2>(a); // three workgroups per CU: 6 tile buffers fit their LDS
