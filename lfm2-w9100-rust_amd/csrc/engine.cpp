@@ -111,7 +111,7 @@ struct Kernels {
     hipModule_t mod = nullptr, pmod = nullptr;
     hipFunction_t split_rows, split_rows_ext, gemm_q6, conv_prefill, rope_kv_prefill, attn_prefill,
         gemm_swiglu, gemm_q6_t32n1, gemm_swiglu_t32, gemm_reduce, attn_merge_split, router_small, router_mfma, router_split, route_topk, route_group, combine_prefill, embed_rows,
-        tile_pack, gemm_q6_n64, gemm_q6_x, gemm_swiglu_x, gemm_q6_t32x, gemm_swiglu_t32x, tile_h16, gemm_h16, gemm_q6_rows,
+        tile_pack, gemm_q6_n64, gemm_q6_x, gemm_swiglu_x, gemm_q6_t32x, gemm_swiglu_t32x, tile_h16, gemm_h16, gemm_q6_rows, gemm_reduce_route4,
         gemm_h16_n64, gemm_swiglu_h16;
     hipFunction_t matvec_long, attn, attn_merge, router, moe_down, argmax, argmax_final, advance,
         dequant, copy, matvec_route, gateup_f, conv_mixer, conv_mixer_r, session_out, session_in, conv_clear, start,
@@ -253,7 +253,8 @@ static int get_kernels(Kernels **out)
                 {&k->gemm_swiglu_x, "k_gemm_q6_swiglu_x"}, {&k->gemm_q6_t32x, "k_gemm_q6_t32x"},
                 {&k->gemm_swiglu_t32x, "k_gemm_q6_swiglu_t32x"}, {&k->tile_h16, "k_q6_tile_h16"},
                 {&k->gemm_h16, "k_gemm_h16"}, {&k->gemm_h16_n64, "k_gemm_h16_n64"},
-                {&k->gemm_swiglu_h16, "k_gemm_swiglu_h16"}, {&k->gemm_q6_rows, "k_gemm_q6_rows"}};
+                {&k->gemm_swiglu_h16, "k_gemm_swiglu_h16"}, {&k->gemm_q6_rows, "k_gemm_q6_rows"},
+                {&k->gemm_reduce_route4, "k_gemm_reduce_route4"}};
     for (auto &f : pfns) {
         e = hipModuleGetFunction(f.f, k->pmod, f.name);
         if (e != hipSuccess) {
@@ -778,7 +779,9 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
         if (router_done)
             *router_done = true;
     }
-    RC(launch(K->gemm_reduce, dim3((g.zrows + 255) / 256, part_rows), 0, s, r));
+    const bool four = r.rw && T >= 128;
+    RC(launch(four ? K->gemm_reduce_route4 : K->gemm_reduce, dim3((g.zrows + 255) / 256, four ? (part_rows + 3) / 4 : part_rows),
+              0, s, r));
     *dispatches += 2;
     return LFM_OK;
 }
