@@ -256,7 +256,7 @@ struct CopyArgs { // plain device copy (achievable-bandwidth reference)
 // ---- prefill (multi-token) path ----------------------------------------------
 // RMSNorm (optional) + binary16 hi/lo split of T rows of K floats, with a per-row
 // power-of-two scale so that |x / scale| < 2^14 (hi/lo then hold ~22 bits).
-// Activations for the small-call GEMMs (calls of up to GEMM_TOKENS tokens) are
+// Activations for the small-call GEMMs are
 // token-blocked: element k of logical row L at
 //   ((L / 32) * (K / 8) + k / 8) * 256 + (L % 32) * 8 + k % 8   (binary16),
 // so the B fragment of 32 rows and 8 k's is 512 contiguous bytes.

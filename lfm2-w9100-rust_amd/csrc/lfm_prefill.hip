@@ -1539,14 +1539,12 @@ k_gemm_swiglu_h16(const GemmArgs a)
     gemm_tiles<true, 4, false, true>(a);
 }
 
-// The same products for calls of up to 128 tokens (chunked prefill: about 8
-// tokens per expert at 64 tokens), 32 tokens per workgroup: a quarter of the
-// padded matrix-core work, and every wave runs on its own.  A lane loads its
-// weight rows' Q6_K bytes a half block ahead and its token column's activation
-// fragments (hi, lo) a stage ahead straight into registers; the block scales
-// are exchanged between lanes by shuffles (lane l holds row l's running scale),
-// so there is no LDS tile and no barrier, and each wave waits only for the
-// loads its next instructions use.  Same arithmetic per (row, token) as
+// The same products for small calls (chunked prefill: about 8 tokens per expert at 64
+// tokens), 32 tokens per workgroup: a quarter of the padded matrix-core work.  A lane
+// loads its weight rows' Q6_K bytes a block ahead into registers; the four waves share
+// the activation tiles (a ring of LDS buffers filled by buffer loads) and meet at a
+// barrier every G stages; the block scales pass between lanes through the wave's own LDS
+// slots (lane l holds row l's running scale).  Same arithmetic per (row, token) as
 // gemm_body.  NI: 32-row tiles per wave (the pair form: its gate and up tile).
 // EXACT: weights in two parts as in gemm_body (the _x kernels).
 // ROWS: the weights come from the row-major planes (Q6Tiles::planes) and each wave finds
@@ -2620,7 +2618,7 @@ extern "C" __global__ __launch_bounds__(WG_THREADS) void k_router_mfma(const Rou
     }
 }
 
-// Router logits for calls of up to 128 tokens: one workgroup per (expert, token)
+// Router logits for small calls without a K split: one workgroup per (expert, token)
 // (grid n_expert x T), thread tid covering inputs 8 tid .. 8 tid + 7 of the
 // token's x . w (dim <= 2048), so the workgroup also sums x^2 for the RMSNorm
 // scale; logits = inv * dot.
