@@ -761,8 +761,7 @@ __device__ __forceinline__ half8 decode_frag(const AChunk &c, uint32_t s, half2v
 // exceed 2048 in magnitude (a binary16 holds every integer up to 2048 only): w the weight
 // rounded to binary16 and r = weight - w, which is 0 or +-1 (the weights are integers of
 // magnitude at most 4096) and which one fused multiply-add forms exactly.  The GEMMs add
-// w xh, r xh and w xl; r xl is left out: |r xl| <= 2^-11 |xh| against a weight above
-// 2048, 2^-22 of the term, the precision of the activations' own split.
+// all four products w xh, r xh, w xl and r xl.
 struct SplitFrag {
     half8 w, r;
 };
@@ -874,11 +873,13 @@ __device__ __forceinline__ void store_rows16(float *out, uint32_t rb, uint32_t z
 }
 
 // EXACT: the weights are formed in two exact parts (decode_frag_split) for any int8
-// scale: three matrix-core products per k-step instead of two (the _x kernels).  The
-// split of the scale into 16 sh + sl that this replaced took four: a block of the model
-// with whole-range scales at 7 / 64 / 512 / 1500 / 3000 tokens 596 / 588 / 1392 / 3165 /
-// 5266 us with four, 570 / 548 / 1286 / 2688 / 4440 us with three; error against 64-bit
-// arithmetic the same (the rest r xl is 2e-8 of a sum over uniform scales and codes).
+// scale: four matrix-core products per k-step instead of two (the _x kernels).  A block of
+// the model with whole-range scales at 7 / 64 / 512 / 1500 tokens takes 406 / 505 / 1130 /
+// 2520 us; with the two parts from the scale (sc = 16 sh + sl, also four products) 407 /
+// 506 / 1156 / 2605 us and an error against 64-bit arithmetic of 2.6e-6 instead of 1.4e-6 at
+// 512 tokens (its parts are of like size, so the sums round more).  Without r xl, 386 /
+// 481 / 1064 / 2270 us: not an option, since where the xh of a row cancel an odd weight
+// above 2048 then counts as its neighbour (4e-4 off).
 // The activation tiles (hi, lo, two buffers) and row factors of a large-call workgroup.
 struct LdsTiles {
     _Float16 *h0, *h1, *l0, *l1;
@@ -1153,6 +1154,9 @@ __device__ __forceinline__ void gemm_body(const GemmArgs &a, const GemmAt &at, u
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].w, bfl[j & 1], acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].r, bfl[j & 1], acc[i][j], 0, 0, 0);
             }
             if (ks < 3) {
 #pragma unroll
@@ -1773,10 +1777,11 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
                 acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i], bcl[kq], acc[i], 0, 0, 0);
             if (ROWS && two) { // uniform
 #pragma unroll
-                for (int i = 0; i < NI; ++i)
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                        decode_frag_rest(A[i][kq & 1], 2 * q + (kq >> 1), ss[i][kq & 1].sc[(kq >> 1) & 1], afc[i]), bch[kq],
-                        acc[i], 0, 0, 0);
+                for (int i = 0; i < NI; ++i) {
+                    const half8 r = decode_frag_rest(A[i][kq & 1], 2 * q + (kq >> 1), ss[i][kq & 1].sc[(kq >> 1) & 1], afc[i]);
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(r, bch[kq], acc[i], 0, 0, 0);
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(r, bcl[kq], acc[i], 0, 0, 0);
+                }
             }
             if (kq < 3) {
 #pragma unroll
@@ -1814,6 +1819,9 @@ __device__ __forceinline__ void gemm_small_body(const GemmArgs &a)
 #pragma unroll
             for (int i = 0; i < NI; ++i)
                 acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].w, bcl[kq], acc[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[i].r, bcl[kq], acc[i], 0, 0, 0);
             if (kq < 3) {
 #pragma unroll
                 for (int i = 0; i < NI; ++i)
