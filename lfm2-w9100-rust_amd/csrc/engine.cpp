@@ -666,10 +666,14 @@ static dim3 gemm_grid(uint32_t rows, uint32_t ntok, uint32_t nz, uint32_t rows_p
 #define SMALL_TOKENS 704u
 // (models narrower than two Q6_K blocks keep to GEMM_TOKENS: their projections
 // cannot be split over K, so no reduce would leave the router partial sums that
-// the expert lists of more than 256 tokens are formed from)
+// the expert lists of more than 256 tokens are formed from; without them the split's
+// route_rows forms the lists)
+static_assert(GEMM_TOKENS <= ROUTE_ROWS_TOKENS, "calls without router partial sums");
 static bool small_call(uint32_t T, uint32_t dim) { return T <= (dim >= 512 ? SMALL_TOKENS : (uint32_t)GEMM_TOKENS); }
 
 #define GEMM_PART_BYTES ((size_t)64 << 20) // split-K partial sums (prefill scratch)
+static_assert(2 * (size_t)SMALL_TOKENS * 2048 * 4 <= GEMM_PART_BYTES,
+              "two slices of an out projection fit, so its reduce can always leave router partial sums");
 #define GEMM_PART_SOFT ((size_t)1600000) // small calls' partial sums, floats (6.4 MB)
 // lfm_q6k_gemm, 6144 x 2048 by 8 / 300 / 1024 tokens: 29 / 60 / 180 us from the planes,
 // 148 / 160 / 240 with the copies; 16384 x 8192 by 2 / 300 / 1024: 64 / 450 / 1290 against
@@ -685,7 +689,7 @@ static bool small_call(uint32_t T, uint32_t dim) { return T <= (dim >= 512 ? SMA
 // then mostly the weight-row tiles and each workgroup's K loop is a chain of
 // dependent stages, so K is split into slices (about 1024 workgroups, each slice
 // at least one Q6_K block, the partials within `part_cap` floats of `part` and
-// within GEMM_PART_SOFT floats) and
+// within GEMM_PART_SOFT floats; with `router` at least two slices, past the latter) and
 // k_gemm_reduce adds the slices in order.  part_rows: output rows the GEMM can
 // write (T, or 4T for expert slots); n_used: ranks per token of the expert slots.
 // `deferred` (non-pair calls): with a K split the reduce is left to the
@@ -739,7 +743,7 @@ static int launch_gemm(Kernels *K, hipStream_t s, GemmArgs g, bool pair, bool sm
         // adding them costs more than the wider grid gains (the 6144-row in_proj at
         // four slices, the dense gate/up pair unsplit, the dense down at twelve)
         S = (uint32_t)std::max<size_t>(1, std::min<size_t>(S, std::min<size_t>(part_cap, GEMM_PART_SOFT) / per));
-        if (router && g.w.nb > 1) // the reduce leaves the router partial sums
+        if (router && g.w.nb > 1 && 2 * per <= part_cap) // the reduce leaves the router partial sums
             S = std::max(S, 2u);
         if (g.y_hi) // the split output is formed in the epilogue from whole sums
             S = 1;
@@ -2272,6 +2276,8 @@ static int pf_ffn(lfm_engine *e, uint32_t l, uint32_t T)
     // with the out projection's router partials (and counts zeroed by its reduce) it
     // routes each token too (no k_route_topk)
     const bool self_route = small && e->pf.router_ready;
+    if (small && !self_route && T > ROUTE_ROWS_TOKENS)
+        return fail(LFM_EINTERNAL, "prefill router: no partial sums for a small call of %u tokens", T);
     if (self_route && rg.nparts > 8) // dim <= 2048 (validate_hparams): at most 8 partials
         return fail(LFM_EINTERNAL, "prefill router: %u partial sums per token > 8", rg.nparts);
     if (!self_route) {

@@ -269,6 +269,7 @@ __host__ __device__ inline size_t blocked_index(uint32_t L, uint32_t k, uint32_t
 #define SPLIT_BLOCKED 1  // blocked, logical row = source row
 #define SPLIT_GROUPED 2  // blocked, logical rows of the expert slots (see SplitArgs)
 
+#define ROUTE_ROWS_TOKENS 256 // the most tokens of a split that forms expert lists without router partial sums
 struct SplitArgs {
     const float *x;      // [T][K]
     const float *norm_w; // nullable

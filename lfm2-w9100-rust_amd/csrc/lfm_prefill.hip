@@ -240,6 +240,7 @@ __device__ __forceinline__ void combine_pieces(const SplitArgs &a, uint32_t t, f
 // earlier tokens that selected e_r (k_route_group's token order), found by every
 // thread i < T testing token i's selection with ballots.  The workgroup also
 // writes its slots' list entries and pos; workgroup 0 writes the counts.
+static_assert(ROUTE_ROWS_TOKENS == WG_THREADS, "route_rows: a token per thread");
 __device__ __forceinline__ uint32_t route_rows(const SplitArgs &a, uint32_t t, uint32_t (&L)[4])
 {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

@@ -88,7 +88,7 @@ def test_real_width_whole_equals_chunks(real, n):
     check_same(hp, n, sw, sc)
 
 
-@pytest.mark.parametrize("n", [2, 33, 200, 750])
+@pytest.mark.parametrize("n", [2, 33, 200, 257, 704, 750])
 @pytest.mark.parametrize("sigma", [0.0, 4.0])
 def test_expert_lists_of_any_length(gpu, oracle, n, sigma):
     """64 experts top-4: a spread of 4 in the selection bias sends every token to the
