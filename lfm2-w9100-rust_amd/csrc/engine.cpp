@@ -675,9 +675,13 @@ static bool small_call(uint32_t T, uint32_t dim) { return T <= (dim >= 512 ? SMA
 static_assert(2 * (size_t)SMALL_TOKENS * 2048 * 4 <= GEMM_PART_BYTES,
               "two slices of an out projection fit, so its reduce can always leave router partial sums");
 #define GEMM_PART_SOFT ((size_t)1600000) // small calls' partial sums, floats (6.4 MB)
-// lfm_q6k_gemm, 6144 x 2048 by 8 / 300 / 1024 tokens: 29 / 60 / 180 us from the planes,
-// 148 / 160 / 240 with the copies; 16384 x 8192 by 2 / 300 / 1024: 64 / 450 / 1290 against
-// 923 / 1070 / 1300 (the two meet there).
+// lfm_q6k_gemm from the planes against the large-call kernels over copies made for the
+// call, in us by 300 / 700 / 1024 tokens: 6144 x 2048 60 / 150 / 172 against 150 / 210 /
+// 227, 16384 x 8192 435 / 906 / 1294 against 1000 / 1176 / 1268.  Weights of 2^28 elements
+// and more meet the copies at fewer tokens (32768 x 8192 at 655, 131072 x 4096 at 480) when
+// the copies' allocations (0.7 GB there) go smoothly, 2350 against 2020 us at 900 tokens of
+// 32768 x 8192; in half the processes those stall for 10-40 ms on every call, so they keep
+// to the planes too.
 #define GEMM_DIRECT_TOKENS 1024u
 #define GEMM_DIRECT_PART ((uint64_t)500000) // its partial sums, floats (2 MB)
 #define GEMM_N64_BELOW 512u // two 128-token workgroups per CU on 256 CUs
@@ -808,9 +812,10 @@ extern "C" int lfm_q6k_gemm(const void *packed, uint64_t rows, uint64_t in_dim, 
     hipStream_t s = (hipStream_t)stream;
     // A call on a weight that is seen once does not pay for copies of it: up to
     // GEMM_DIRECT_TOKENS tokens k_gemm_q6_rows reads the planes (small-call kernel:
-    // activations token-blocked, rows padded to 32), one wait and no device allocation of
-    // 2 MB or more for ordinary sizes (those take 35 us each to make and free).  Beyond,
-    // the large-call kernels over a tile copy and a binary16 copy.
+    // activations token-blocked, rows padded to 32), with one wait.  An allocation of 2 MB
+    // or more takes 35 us to make and free: the activations' two halves reach that at 512
+    // tokens of 2048 inputs.  Beyond, the large-call kernels over a tile copy and a binary16
+    // copy.
     const bool direct = T <= GEMM_DIRECT_TOKENS;
     const size_t hrows = direct ? (T + 31) / 32 * 32 : T;
     uint16_t *hi = nullptr, *lo = nullptr;
