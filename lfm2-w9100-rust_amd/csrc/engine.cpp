@@ -1718,9 +1718,16 @@ extern "C" int lfm_engine_finalize(lfm_engine *e)
                                                "ffn_up.weight",            "ffn_down.weight",
                                                "ffn_gate_exps.weight",     "ffn_up_exps.weight",
                                                "ffn_down_exps.weight"};
+    // (of the last layer only q / k / v and in_proj, the latter for the small-call kernels:
+    // three rows go through it, and the one row left after the mixer through the decode
+    // step's kernels)
+    const std::string last = "blk." + std::to_string(hp.n_layers - 1) + ".";
     for (auto &kv : e->tensors) {
         DevTensor &t = kv.second;
         const size_t n = kv.first.size();
+        const bool in_last = kv.first.compare(0, last.size(), last) == 0;
+        if (in_last && !ends_with(kv.first, "shortconv.in_proj.weight"))
+            continue;
         bool gemm = false;
         for (const char *suf : gemm_weights) {
             const size_t m = strlen(suf);
@@ -1733,7 +1740,7 @@ extern "C" int lfm_engine_finalize(lfm_engine *e)
             // and their decode in registers measured faster (the other weights are
             // read by several token tiles through the caches)
             const bool pair_exps = ends_with(kv.first, "ffn_gate_exps.weight") || ends_with(kv.first, "ffn_up_exps.weight");
-            if (!pair_exps)
+            if (!pair_exps && !in_last)
                 RC(make_h16(e->K, e->stream, &t.tiles, &t.h16_dev));
         }
         // router rows for the large calls' matrix-core router: w * 2^s in binary16

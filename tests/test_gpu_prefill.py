@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from conftest import rel_l2
-from model_util import gpu_engine, model_tensors, oracle_engine, top2_margin
+from model_util import gpu_engine, model_tensors, oracle_engine, small_hparams, top2_margin
 
 pytestmark = pytest.mark.gpu
 
@@ -292,3 +292,20 @@ def test_forward_token_after_halted_decode(gpu, real_width):
     g.reset_session()
     lg = g.forward(prompt, 0)
     assert int(np.argmax(lg)) == tok and np.float32(lg.max()).tobytes() == np.float32(val).tobytes()
+
+
+@pytest.mark.parametrize("kinds", [("conv",), ("attn",), ("conv", "attn"), ("attn", "conv", "conv")])
+def test_h16_copies_only_where_large_calls_read_them(gpu, kinds):
+    """binary16 copies: every projection of the layers before the last (dense FFNs here),
+    and of the last one q / k / v, which all its rows pass."""
+    hp = small_hparams(kinds=kinds, dense_lead=len(kinds))
+    g = gpu_engine(hp, model_tensors(hp), ctx=64)
+    dim, qkv = hp.dim, hp.dim + 2 * 64 * 2
+    want = 0
+    for i, kind in enumerate(kinds):
+        if i + 1 < len(kinds):
+            want += (4 * dim if kind == "conv" else qkv + dim) + 3 * hp.n_ff
+        else:
+            want += qkv if kind == "attn" else 0
+    assert g.h16_bytes() == 2 * dim * want
+    g.close()
