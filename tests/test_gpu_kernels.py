@@ -106,18 +106,17 @@ def test_argmax_cases(gpu, oracle):
                                            (2048, 7168, 64), (256, 1792, 1), (2048, 2048, 31),
                                            (512, 1024, 32), (6144, 2048, 33), (1792, 2048, 128),
                                            (1000, 512, 150), (1000, 512, 40), (8192, 256, 2048),
-                                           (3072, 2048, 64), (3200, 512, 64)])
+                                           (3072, 2048, 64), (3200, 512, 64), (130, 768, 1025),
+                                           (1000, 512, 1290), (6144, 2048, 1100)])
 def test_gemm_prefill_matches_f64(gpu, oracle, rows, in_dim, T):
     """Matrix-core GEMM (binary16 sc*(q-32) weights, hi/lo activations, fp32 d
-    scaling) against the f64 q6k_matvec oracle per token: rel-L2 <= 1e-5.  Calls
-    of up to 128 tokens read token-blocked activations (32-row tiles), so the
-    tokens on either side of a tile edge are checked too.  The weights are read
-    from a copy in 32-row tiles whose rows past the matrix are zero: 130 and
-    1000 rows end inside a tile, with both the large-call and the 32-token tiles.
-    Large calls run 64-token tiles when 128-token ones would make fewer than 512
-    workgroups: 8192 rows x 2048 tokens is the case that runs the 128-token tiles.
-    Small calls of up to 3072 rows run one 32-row tile per wave (3072 rows), wider
-    ones two (3200)."""
+    scaling) against the f64 q6k_matvec oracle per token: rel-L2 <= 1e-5.  Calls of up
+    to 1024 tokens read the weight's planes and token-blocked activations (32-row tiles,
+    one per wave), so the tokens on either side of a tile edge are checked too; K is
+    split where few workgroups would run.  Larger calls read copies in 32-row tiles whose
+    rows past the matrix are zero (130 and 1000 rows end inside a tile) and run 64-token
+    tiles when 128-token ones would make fewer than 512 workgroups: 8192 rows x 2048
+    tokens is the case that runs the 128-token tiles."""
     raw = blocks(rows * in_dim // 256, rows * 7 + T).reshape(-1)
     rng = np.random.default_rng(T)
     x = rng.standard_normal((T, in_dim)).astype(np.float32)
@@ -131,13 +130,17 @@ def test_gemm_prefill_matches_f64(gpu, oracle, rows, in_dim, T):
 
 
 @pytest.mark.parametrize("rows,in_dim,T", [(6144, 2048, 200), (1792, 2048, 129), (8192, 256, 2048),
-                                           (1000, 512, 150), (2048, 7168, 300)])
+                                           (1000, 512, 150), (2048, 7168, 300),
+                                           (6144, 2048, 1100), (1000, 512, 1290), (2048, 7168, 1056),
+                                           (8192, 1024, 2048)])
 def test_gemm_prefill_h16_copy_bit_identical(gpu, oracle, monkeypatch, rows, in_dim, T):
-    """Large calls read the weights from a binary16 fragment copy made once
+    """Calls of more than 1024 tokens read the weights from a binary16 fragment copy
     (k_q6_tile_h16: the A fragments the Q6_K kernels decode in registers, k-step
     by k-step); with LFM_PREFILL_H16=0 they decode Q6_K in registers instead.  The
     two paths run the same products in the same order, so their outputs agree
-    bit for bit; both stay within 1e-5 of the f64 oracle."""
+    bit for bit, over one block and over 28, with 64-token tiles and (8192 rows x 2048
+    tokens) 128-token ones; both stay within 1e-5 of the f64 oracle.  Smaller calls read
+    the planes whatever the setting."""
     raw = blocks(rows * in_dim // 256, rows * 5 + T).reshape(-1)
     x = np.random.default_rng(T + 1).standard_normal((T, in_dim)).astype(np.float32)
     x[1] *= 1000.0
@@ -150,19 +153,10 @@ def test_gemm_prefill_h16_copy_bit_identical(gpu, oracle, monkeypatch, rows, in_
         assert rel_l2(y_h16[t], oracle.q6k_matvec(raw, in_dim, rows, x[t])) <= 1e-5
 
 
-@pytest.mark.parametrize("T", [130, 64, 5])
-def test_gemm_prefill_block_scale_edges(gpu, oracle, T):
-    """Super-block scales d that are zero (first, last, every other or every
-    block of a row), -0.0, subnormal, or spread over eleven decades within one
-    row: the GEMM folds d into its accumulators block by block, so every row
-    is checked on its own against the f64 oracle (rel-L2 over tokens <= 1e-5;
-    rows whose blocks all have d = 0 give exactly 0).  T = 130 runs the 128-token
-    tiles; T <= 128 the split-K path with 32-token tiles, whose waves exchange the
-    scales by lane shuffles."""
-    rows, in_dim = 300, 2048
-    nb = in_dim // 256
-    raw = blocks(rows * nb, 77).reshape(rows, nb, 210)
-    rng = np.random.default_rng(5)
+def edge_scales(rows, nb, rng):
+    """Super-block scales d [rows][nb] by kind = row % 8: zero in every block (0), the
+    first (1), the last (2) or every other one (3), spread over eleven decades with
+    subnormal ones among them (4), -0.0 in every third (5), ordinary (6, 7)."""
     d = (rng.standard_normal((rows, nb)) * 1e-3).astype(np.float16)
     kind = np.arange(rows) % 8
     d[kind == 0] = 0
@@ -173,6 +167,25 @@ def test_gemm_prefill_block_scale_edges(gpu, oracle, T):
     mag = 10.0 ** rng.uniform(-7, 4.5, size=(int(spread.sum()), nb))
     d[spread] = (mag * rng.choice([-1.0, 1.0], size=mag.shape)).astype(np.float16)
     d[kind == 5, 1::3] = np.float16(-0.0)
+    return d, kind
+
+
+@pytest.mark.parametrize("T,h16,sc_lim", [(130, "1", 32), (64, "1", 32), (5, "1", 32), (130, "1", 128), (5, "1", 128),
+                                          (1100, "1", 32), (1100, "0", 32), (1100, "1", 128)])
+def test_gemm_prefill_block_scale_edges(gpu, oracle, monkeypatch, T, h16, sc_lim):
+    """Super-block scales d that are zero (first, last, every other or every
+    block of a row), -0.0, subnormal, or spread over eleven decades within one
+    row: the GEMM folds d into its accumulators block by block, so every row
+    is checked on its own against the f64 oracle (rel-L2 over tokens <= 1e-5;
+    rows whose blocks all have d = 0 give exactly 0).  T <= 1024 reads the planes
+    (split K, 32-token tiles), 1100 the binary16 copies or the Q6_K tile copies
+    (h16 0); sc_lim 128: the two-part weights."""
+    monkeypatch.setenv("LFM_PREFILL_H16", h16)
+    rows, in_dim = 300, 2048
+    nb = in_dim // 256
+    raw = blocks(rows * nb, 77, sc_lim=sc_lim).reshape(rows, nb, 210)
+    rng = np.random.default_rng(5)
+    d, kind = edge_scales(rows, nb, rng)
     raw[:, :, 208:210] = d.view(np.uint8).reshape(rows, nb, 2)
     raw = raw.reshape(-1)
     x = rng.standard_normal((T, in_dim)).astype(np.float32)
@@ -186,15 +199,16 @@ def test_gemm_prefill_block_scale_edges(gpu, oracle, T):
         assert err <= 1e-5, (r, kind[r], err)
 
 
-@pytest.mark.parametrize("T,synth", [(130, False), (64, False), (200, True), (64, True), (1, True)])
+@pytest.mark.parametrize("T,synth", [(130, False), (64, False), (200, True), (64, True), (1, True), (1100, False),
+                                     (1100, True)])
 def test_gemm_prefill_full_int8_scales(gpu, oracle, T, synth):
     """Sub-block scales over the whole int8 range (uniform int8, or the synthetic
     full-scale blocks: [-127, 127] with one -128 per super-block, as ggml's
     quantizer writes them).  A binary16 holds sc * (q - 32) exactly only up to
-    magnitude 2048, so weights with such scales (the tile copy flags them) run
-    the split-scale kernels, sc = (sc & ~15) + (sc & 15), both partial weights
-    exact: against the f64 oracle the 1e-5 bar holds as for small scales.
-    T = 200 runs the large-call kernel, T = 64 and 1 the small-call ones."""
+    magnitude 2048, so weights with such scales are added in two exact parts, the
+    weight rounded to binary16 and its remainder: against the f64 oracle the 1e-5 bar
+    holds as for small scales.  T <= 1024 reads the planes (each wave looks at its half
+    block's scales), T = 1100 the tile copy, which is flagged as a whole."""
     rows, in_dim = 1024, 2048
     if synth:
         raw = gpu.synth_q6k_blocks(93, "full.weight", rows * in_dim // 256, full_scales=True)
@@ -234,10 +248,9 @@ def test_gemm_prefill_weights_exact(gpu, oracle, T, k0, lo, hi):
     rows hold every (scale, code) pair of the range; token t is the one-hot vector
     of column k0 + t, so y[t][r] is weight (r, k0 + t) times 1 with nothing else
     added, and must equal sc (q - 32) exactly.  Scales within [-64, 64] keep every
-    product within binary16's exact integers (the default kernels); the whole int8
-    range runs the split-scale kernels.  The encoding is checked against the
-    oracle's dequant first.  T = 256 runs the large-call kernels, T <= 128 the
-    32-token tiles."""
+    product within binary16's exact integers (one part); the whole int8 range needs the
+    two-part weights.  The encoding is checked against the oracle's dequant first.  All
+    of these read the planes (the copies: test_gpu_gemm_planes.py)."""
     rows, in_dim = 256, 256
     k = np.arange(in_dim)
     codes = (k[None, :] + np.arange(rows)[:, None]) % 64

@@ -59,9 +59,10 @@ def check_prefill(gpu, oracle, hp, tensors, n, ctx):
 @pytest.mark.parametrize("n", [70, 200])
 def test_prefill_wide_router(gpu, oracle, n):
     """48 experts top-4: the prefill routers' paths for more than 32 experts (at 70
-    tokens the small call's; at 200 the large call's matrix-core router, whose second
-    pass covers experts 32..47)."""
-    hp = gpu.make_hparams(dim=256, heads=4, n_layers=2, attention_layers=(1,), kv=2, vocab=500,
+    tokens the small call's; at 200, a large call at this width, the matrix-core router,
+    whose second pass covers experts 32..47), in two layers before the last, whose one
+    row the decode step's router takes."""
+    hp = gpu.make_hparams(dim=256, heads=4, n_layers=4, attention_layers=(1,), kv=2, vocab=500,
                           eos=1 << 30, n_expert=48, n_used=4, expert_ff=256, n_ff=512,
                           dense_lead=1)
     tensors = model_tensors(hp, gpu.synth_opts(0x5EED, bias_sigma=0.1))
@@ -74,12 +75,13 @@ def test_prefill_real_width(gpu, oracle, real_width, n):
     check_prefill(gpu, oracle, hp, tensors, n, ctx=512)
 
 
-@pytest.mark.parametrize("n", [100, 128, 129, 400])
+@pytest.mark.parametrize("n", [100, 128, 129, 400, 720])
 def test_prefill_crowded_experts(gpu, oracle, crowded, n):
-    """8 experts top-2: at 100 and 128 tokens (small calls) experts hold more than one
-    32-row tile of gathered activations; at 129 and 400 the large-call kernels run."""
+    """8 experts top-2: up to 704 tokens (small calls) experts hold several 32-row tiles
+    of gathered activations; at 720 the large-call kernels run, with several 128-token
+    tiles per expert."""
     hp, tensors = crowded
-    check_prefill(gpu, oracle, hp, tensors, n, ctx=512)
+    check_prefill(gpu, oracle, hp, tensors, n, ctx=768)
 
 
 def test_prefill_chunks_then_decode(gpu, oracle, real_width):
@@ -115,8 +117,7 @@ def test_prefill_chunks_then_decode(gpu, oracle, real_width):
 
 def test_prefill_64_token_chunks(gpu, oracle, real_width):
     """A 448-token prompt in 64-token chunks (api_stream.rs:57-63, work_bound.rs
-    PREFILL_CHUNK): calls of up to 128 tokens take the split-K GEMM with 32-token
-    tiles, and chunks from position 192 on split attention over key ranges.  The
+    PREFILL_CHUNK): they take the split-K GEMM with 32-token tiles, and chunks from position 192 on split attention over key ranges.  The
     last logits and the resident state match the oracle and the engine's own
     whole-prompt forward."""
     hp, tensors = real_width
@@ -145,41 +146,42 @@ def test_prefill_chunks_repeat_bit_exact(gpu, real_width):
     """Small calls take each token's slot in its experts' lists with an atomic add,
     so a token's row may sit elsewhere in its expert's tile from one run to the
     next; what is computed for it must not change: two engines prefilling the
-    same 192 tokens in 64-token calls, then 300 more in one large call, give
-    bit-identical logits and state."""
+    same 192 tokens in 64-token calls, then 300 more in one small call and 720 in a
+    large one, give bit-identical logits and state."""
     hp, tensors = real_width
-    prompt = [int(t) for t in np.random.default_rng(17).integers(0, hp.vocab, 492)]
+    prompt = [int(t) for t in np.random.default_rng(17).integers(0, hp.vocab, 1212)]
     outs = []
     for _ in range(2):
-        g = gpu_engine(hp, tensors, ctx=512)
+        g = gpu_engine(hp, tensors, ctx=1216)
         for s in range(0, 192, 64):
             lg = g.forward(prompt[s:s + 64], s)
-        lw = g.forward(prompt[192:], 192)
-        outs.append((lg.view(np.uint32).copy(), np.frombuffer(g.snapshot_resident_cache(192), np.uint32).copy(),
-                     lw.view(np.uint32).copy(), np.frombuffer(g.snapshot_resident_cache(492), np.uint32).copy()))
+        out = [lg.view(np.uint32).copy(), np.frombuffer(g.snapshot_resident_cache(192), np.uint32).copy()]
+        for a, b in ((192, 492), (492, 1212)):
+            lw = g.forward(prompt[a:b], a)
+            out += [lw.view(np.uint32).copy(), np.frombuffer(g.snapshot_resident_cache(b), np.uint32).copy()]
+        outs.append(out)
         g.close()
     for a, b in zip(outs[0], outs[1]):
         assert np.array_equal(a, b)
 
 
 def test_prefill_mixed_chunk_sizes(gpu, oracle, real_width):
-    """One prompt in calls of 1, 127, 128, 129, 3 and 92 tokens: both sides of the
-    128-token line between the split-K small-call GEMMs (one 32-row tile per wave up
-    to 3072 rows, partial sums capped) and the large-call ones (64-token tiles for
-    grids under 512 workgroups, which every projection here is), each call reading
-    the KV and conv state the previous ones left.  The last logits and the resident
-    state match the oracle's token-by-token forward and the engine's whole-prompt
-    call."""
+    """One prompt in calls of 1, 127, 128, 129, 3, 92 and 705 tokens: small calls (split-K
+    GEMMs, one 32-row tile per wave; router partials for four tokens per workgroup from
+    128 tokens on) and a large one (64-token tiles for grids under 512 workgroups, which
+    every projection here is), each reading the KV and conv state the previous ones left.
+    The last logits and the resident state match the oracle's token-by-token forward and
+    the engine's whole-prompt call."""
     hp, tensors = real_width
-    sizes = [1, 127, 128, 129, 3, 92]
+    sizes = [1, 127, 128, 129, 3, 92, 705]
     n = sum(sizes)
     prompt = [int(t) for t in np.random.default_rng(23).integers(0, hp.vocab, n)]
-    g = gpu_engine(hp, tensors, ctx=512)
+    g = gpu_engine(hp, tensors, ctx=1216)
     s = 0
     for c in sizes:
         lg = g.forward(prompt[s:s + c], s)
         s += c
-    o = oracle_engine(oracle, hp, tensors, ctx=512)
+    o = oracle_engine(oracle, hp, tensors, ctx=1216)
     lo = o.forward(prompt, 0)
     err = rel_l2(lg, lo)
     sg = np.frombuffer(g.snapshot_resident_cache(n), np.float32)
@@ -188,17 +190,18 @@ def test_prefill_mixed_chunk_sizes(gpu, oracle, real_width):
     print(f"mixed chunks {sizes}: logits rel-L2 {err:.3e}, state rel-L2 {serr:.3e}")
     assert err <= 1e-3
     assert serr <= 1e-3
-    w = gpu_engine(hp, tensors, ctx=512)
+    w = gpu_engine(hp, tensors, ctx=1216)
     lw = w.forward(prompt, 0)
     assert rel_l2(lg, lw) <= 1e-3
 
 
-def test_prefill_full_int8_scales_model(gpu, oracle):
+@pytest.mark.parametrize("n", [300, 720])
+def test_prefill_full_int8_scales_model(gpu, oracle, n):
     """A real-width model whose Q6_K weights use the whole int8 scale range, as
     model files do (synthetic full_scales: one sub-block per super-block at -128).
-    Its GEMMs take the split-scale kernels, so the whole-prompt call (large-call
-    kernels, 300 tokens) and the same prompt in 64-token calls (small-call
-    kernels) stay as close to the decode graph's stepwise forward (weights formed
+    Its GEMMs take the two-part kernels, so the whole-prompt call (300 tokens:
+    small-call kernels, 720: large-call ones) and the same prompt in 64-token calls
+    stay as close to the decode graph's stepwise forward (weights formed
     in fp32) as the synthetic model's prefill does, and match the oracle."""
     hp = gpu.make_hparams(dim=2048, heads=32, n_layers=4, attention_layers=(1, 3), kv=8,
                           vocab=4096, eos=1 << 30, n_expert=32, n_used=4, expert_ff=1792,
@@ -207,9 +210,8 @@ def test_prefill_full_int8_scales_model(gpu, oracle):
     raw = next(d for nm, _, _, d in tensors if nm == "blk.1.ffn_gate_exps.weight")
     sc = raw.reshape(-1, 210)[:, 192:208].view(np.int8)
     assert sc.min() == -128 and np.abs(sc.astype(int)).max() == 128
-    n = 300
     prompt = [int(t) for t in np.random.default_rng(31).integers(0, hp.vocab, n)]
-    g = gpu_engine(hp, tensors, ctx=512)
+    g = gpu_engine(hp, tensors, ctx=768)
     lw = g.forward(prompt, 0)
     sw = np.frombuffer(g.snapshot_resident_cache(n), np.float32)
     g.reset_session()
@@ -222,7 +224,7 @@ def test_prefill_full_int8_scales_model(gpu, oracle):
     ls = g.forward(prompt, 0)
     ss = np.frombuffer(g.snapshot_resident_cache(n), np.float32)
     g.close()
-    o = oracle_engine(oracle, hp, tensors, ctx=512)
+    o = oracle_engine(oracle, hp, tensors, ctx=768)
     lo = o.forward(prompt, 0)
     so = np.frombuffer(o.snapshot(n), np.float32)
     o.close()
@@ -238,20 +240,22 @@ def test_prefill_full_int8_scales_model(gpu, oracle):
         assert e[k][0] <= 1e-3 and e[k][1] <= 1e-3, (k, e[k])
 
 
-def test_prefill_h16_copy_matches_q6_decode(gpu, real_width, monkeypatch):
+@pytest.mark.parametrize("n", [300, 705, 1000])
+def test_prefill_h16_copy_matches_q6_decode(gpu, real_width, monkeypatch, n):
     """The whole prompt with the large-call GEMMs on the binary16 fragment copies
     (the default) and with LFM_PREFILL_H16=0 (Q6_K decoded in registers, no copies
     made at finalize): logits and resident state bit-identical, at real widths
-    (in_proj, out/o projections, q/k/v, dense and expert gate/up/down)."""
+    (in_proj, out/o projections, q/k/v, dense gate/up/down and the experts' down).
+    300 tokens run the small-call kernels, which read neither copy."""
     hp, tensors = real_width
-    prompt = [int(t) for t in np.random.default_rng(11).integers(0, hp.vocab, 300)]
-    g = gpu_engine(hp, tensors, ctx=512)
+    prompt = [int(t) for t in np.random.default_rng(11).integers(0, hp.vocab, n)]
+    g = gpu_engine(hp, tensors, ctx=1024)
     assert g.h16_bytes() > 0
     lg = g.forward(prompt, 0)
     sg = g.snapshot_resident_cache(len(prompt))
     g.close()
     monkeypatch.setenv("LFM_PREFILL_H16", "0")
-    q = gpu_engine(hp, tensors, ctx=512)
+    q = gpu_engine(hp, tensors, ctx=1024)
     assert q.h16_bytes() == 0
     lq = q.forward(prompt, 0)
     sq = q.snapshot_resident_cache(len(prompt))

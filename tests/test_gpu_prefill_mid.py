@@ -64,7 +64,7 @@ def test_boundary_matches_oracle(gpu, oracle, n):
 @pytest.fixture(scope="module", params=[0, 1], ids=["narrow", "full_scales"])
 def real(gpu, request):
     """Real widths, one layer of each kind, sub-block scales within [-32, 31] or over
-    the whole int8 range (the split-scale kernels)."""
+    the whole int8 range (the two-part kernels)."""
     hp = gpu.make_hparams(dim=2048, heads=32, n_layers=4, attention_layers=(2,), kv=8, vocab=4096,
                           eos=1 << 30, n_expert=32, n_used=4, expert_ff=1792, n_ff=7168, dense_lead=1)
     e = gpu.GpuEngine.load_synthetic(hp, gpu.synth_opts(0x5EED, full_scales=request.param), ctx=1024)
@@ -114,8 +114,8 @@ def test_expert_lists_of_any_length(gpu, oracle, n, sigma):
 def test_last_columns_of_large_calls(gpu, oracle, monkeypatch, n, full_scales, h16):
     """Large-call kernels (a model narrower than 512 runs them from 129 tokens) with 1, 32,
     33, 65, 97 and 128 columns in the last 128-token tile: each form of the last tile, and
-    the experts' own list ends, for the binary16 copies, the Q6_K weights and the two-part
-    weights."""
+    the experts' own list ends, for the binary16 copies, the Q6_K weights (bit for bit what
+    the copies give) and the two-part weights."""
     monkeypatch.setenv("LFM_PREFILL_H16", h16)
     hp = gpu.make_hparams(dim=256, heads=4, n_layers=4, attention_layers=(1,), kv=2, vocab=1000,
                           eos=1 << 30, n_expert=8, n_used=4, expert_ff=256, n_ff=512, dense_lead=1)
@@ -124,6 +124,13 @@ def test_last_columns_of_large_calls(gpu, oracle, monkeypatch, n, full_scales, h
     g = gpu_engine(hp, tensors, ctx=256)
     o = oracle_engine(oracle, hp, tensors, ctx=256)
     lg, lo = g.forward(prompt, 0), o.forward(prompt, 0)
+    sg = state(g, n)
     assert rel_l2(lg, lo) <= 1e-3
-    assert rel_l2(state(g, n), np.frombuffer(o.snapshot(n), np.float32)) <= 1e-3
+    assert rel_l2(sg, np.frombuffer(o.snapshot(n), np.float32)) <= 1e-3
     g.close()
+    if h16 == "0":
+        monkeypatch.setenv("LFM_PREFILL_H16", "1")
+        g = gpu_engine(hp, tensors, ctx=256)
+        assert g.h16_bytes() > 0
+        assert g.forward(prompt, 0).tobytes() == lg.tobytes() and state(g, n).tobytes() == sg.tobytes()
+        g.close()
