@@ -145,7 +145,7 @@ def matvec_roofline(iters=200):
 def full_scale_prefill(hp, prompt):
     """The same prompt through a model whose Q6_K sub-block scales span the whole
     int8 range with one -128 per super-block, as model files have them: its GEMMs
-    run the split-scale kernels (exact binary16 weights for every scale)."""
+    run the two-part kernels (exact weights for every scale)."""
     e = lfm_hip.GpuEngine.load_synthetic(hp, lfm_hip.synth_opts(SEED, full_scales=1), ctx=CTX,
                                          threads=16)
     e.forward(prompt[:256], 0)  # untimed: first launches
@@ -170,7 +170,7 @@ def full_scale_prefill(hp, prompt):
             "chunked_ms": round(chunked * 1e3, 1),
             "next_token_equals_whole_prompt": nxt == int(np.argmax(logits)),
             "note": "synthetic weights with int8 sub-block scales over the whole range (one -128 per "
-                    "super-block): the GEMMs run the split-scale kernels, four matrix-core passes "
+                    "super-block): the GEMMs run the two-part kernels, four matrix-core passes "
                     "per product"}
 
 

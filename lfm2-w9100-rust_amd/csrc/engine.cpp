@@ -657,12 +657,16 @@ static dim3 gemm_grid(uint32_t rows, uint32_t ntok, uint32_t nz, uint32_t rows_p
 }
 
 // Calls of up to SMALL_TOKENS tokens run the small-call kernels (token-blocked
-// activations, 32-token tiles, split K): a 4-layer block of the model (one layer of
-// each kind) at 129 / 203 / 512 / 700 tokens takes 0.70 / 0.76 / 1.09 / 1.38 ms against
-// 1.23 / 1.24 / 1.26 / 1.43 ms with the large-call kernels, whose 128-token tiles leave
-// most CUs idle (a 2048-row projection of 203 tokens is 32 workgroups) and most of an
-// expert's tile empty; with whole-range int8 scales 0.68 / 0.83 / 1.32 / 1.64 ms against
-// 1.44 / 1.48 / 1.75 / 1.99.  At 1024 tokens the two meet (1.72 against 1.67 ms).
+// activations, 32-token tiles, split K): the large-call kernels' 128-token tiles leave
+// most CUs idle there (a 2048-row projection of 203 tokens is 32 workgroups) and most of
+// an expert's tile empty.  A 4-layer block of the model (one layer of each kind) at 130 /
+// 203 / 350 / 512 / 704 tokens takes 0.50 / 0.58 / 0.79 / 0.95 / 1.18 ms with them and
+// 0.87 / 0.93 / 1.01 / 1.11 / 1.31 ms with the large-call kernels; with whole-range int8
+// scales 0.59 / 0.69 / 0.95 / 1.13 / 1.45 against 1.13 / 1.23 / 1.36 / 1.50 / 1.73 ms; at
+// width 1024 (32 experts of 512) 0.29 / 0.31 / 0.36 / 0.43 / 0.49 against 0.52 / 0.56 / 0.56
+// / 0.65 / 0.69 ms.  Narrow scales at width 2048 meet at about 1000 tokens (0.99-1.04 from
+// 900 to 1100), whole-range ones at 1400, narrower models beyond; the line lies below all
+// of them (the small calls' scratch grows with it, 0.5 MB a token for the model's experts).
 #define SMALL_TOKENS 704u
 // (models narrower than two Q6_K blocks keep to GEMM_TOKENS: their projections
 // cannot be split over K, so no reduce would leave the router partial sums that

@@ -822,30 +822,6 @@ extern "C" __global__ __launch_bounds__(64) void k_q6_tile_h16(const TileH16Args
     }
 }
 
-// C[n][row] (+)= sum_k W[row][k] * X[n][k] for weight rows [0, zrows) of group
-// z and token columns n < ntok.  Column n reads activation row (tok ? tok[n] :
-// n) and writes output row (slot ? slot[n] : n).  The pair form (k_gemm_q6_swiglu)
-// multiplies the gate weight w and the up weight w2 by the same activations and
-// writes silu(gate) * up (lfm.rs:578-582 SwiGLU, g / (1 + e^-g) * u).
-//
-// A workgroup computes 256 weight rows x 128 tokens (32 NJ): wave w owns rows 64w..64w+63
-// for all 128 tokens (2 x 4 tiles of v_mfma_f32_32x32x16_f16, hi and lo
-// activation halves); in the pair form its two row tiles are the same 32 rows of
-// the gate and of the up weight (128 rows of each per workgroup), so a lane holds
-// a row's gate and up sums side by side.  K advances in 64-wide stages:
-//   * weights never touch LDS: each lane loads its rows' Q6_K bytes one half
-//     block ahead into registers and decodes the MFMA A fragments itself, the
-//     next k-step's fragments while the current k-step's MFMAs run;
-//   * activation tiles go global -> LDS directly (buffer_load_dwordx4 ... lds),
-//     double-buffered, one barrier per stage;
-//   * the super-block scale d is folded into the accumulators: they hold
-//     sum_b d_b P_b / u with u the last nonzero d seen, so entering block b
-//     multiplies them by u / d_b (blocks with d = 0 contribute zero weights),
-//     and the epilogue multiplies by the final u.
-// Tiles are handed out so that each XCD takes a contiguous run with the weight rows
-// fastest (GemmAt), and the workgroups resident on one XCD share activation tiles in
-// its L2.  With ksplit > 1 a workgroup runs its slice's blocks only and writes its
-// sums to part, which k_gemm_reduce adds up in slice order.
 // A lane's 16 accumulator rows of a 32-row tile are rb + 8 (e / 4) + e % 4 (rb =
 // the tile's first row + 4 p).  Writes v (add false) or adds it (add true) to those
 // rows of out below zrows.  With every row in range the old values are read in one
@@ -873,14 +849,6 @@ __device__ __forceinline__ void store_rows16(float *out, uint32_t rb, uint32_t z
     }
 }
 
-// EXACT: the weights are formed in two exact parts (decode_frag_split) for any int8
-// scale: four matrix-core products per k-step instead of two (the _x kernels).  A block of
-// the model with whole-range scales at 7 / 64 / 512 / 1500 tokens takes 406 / 505 / 1130 /
-// 2520 us; with the two parts from the scale (sc = 16 sh + sl, also four products) 407 /
-// 506 / 1156 / 2605 us and an error against 64-bit arithmetic of 2.6e-6 instead of 1.4e-6 at
-// 512 tokens (its parts are of like size, so the sums round more).  Without r xl, 386 /
-// 481 / 1064 / 2270 us: not an option, since where the xh of a row cancel an odd weight
-// above 2048 then counts as its neighbour (4e-4 off).
 // The activation tiles (hi, lo, two buffers) and row factors of a large-call workgroup.
 struct LdsTiles {
     _Float16 *h0, *h1, *l0, *l1;
@@ -949,6 +917,40 @@ __device__ __forceinline__ GemmAt gemm_at_group(const GemmArgs &a, uint32_t gx, 
     return w;
 }
 
+// C[n][row] (+)= sum_k W[row][k] * X[n][k] for weight rows [0, zrows) of group
+// z and token columns n < ntok.  Column n reads activation row (tok ? tok[n] :
+// n) and writes output row (slot ? slot[n] : n).  The pair form (k_gemm_q6_swiglu)
+// multiplies the gate weight w and the up weight w2 by the same activations and
+// writes silu(gate) * up (lfm.rs:578-582 SwiGLU, g / (1 + e^-g) * u).
+//
+// A workgroup computes 256 weight rows x 32 NJ tokens (128 in the widest form): wave w
+// owns rows 64w..64w+63 for all of them (2 x NJ tiles of v_mfma_f32_32x32x16_f16, hi and
+// lo activation halves); in the pair form its two row tiles are the same 32 rows of
+// the gate and of the up weight (128 rows of each per workgroup), so a lane holds
+// a row's gate and up sums side by side.  K advances in 64-wide stages:
+//   * weights never touch LDS: each lane loads its rows' Q6_K bytes one half
+//     block ahead into registers and decodes the MFMA A fragments itself, the
+//     next k-step's fragments while the current k-step's MFMAs run;
+//   * activation tiles go global -> LDS directly (buffer_load_dwordx4 ... lds),
+//     double-buffered, one barrier per stage;
+//   * the super-block scale d is folded into the accumulators: they hold
+//     sum_b d_b P_b / u with u the last nonzero d seen, so entering block b
+//     multiplies them by u / d_b (blocks with d = 0 contribute zero weights),
+//     and the epilogue multiplies by the final u.
+// Tiles are handed out so that each XCD takes a contiguous run with the weight rows
+// fastest (GemmAt), and the workgroups resident on one XCD share activation tiles in
+// its L2.  With ksplit > 1 a workgroup runs its slice's blocks only and writes its
+// sums to part, which k_gemm_reduce adds up in slice order.
+//
+// EXACT: the weights are formed in two exact parts (decode_frag_split) for any int8
+// scale: four matrix-core products per k-step instead of two (the _x kernels).  A block of
+// the model with whole-range scales at 7 / 64 / 512 / 1500 tokens takes 406 / 505 / 1130 /
+// 2520 us; with the two parts from the scale (sc = 16 sh + sl, also four products) 407 /
+// 506 / 1156 / 2605 us and an error against 64-bit arithmetic of 2.6e-6 instead of 1.4e-6 at
+// 512 tokens (its parts are of like size, so the sums round more).  Without r xl, 386 /
+// 481 / 1064 / 2270 us: not an option, since where the xh of a row cancel an odd weight
+// above 2048 then counts as its neighbour (4e-4 off).
+//
 // NJ: 32-column token tiles that the workgroup computes, from column n0 (a kernel of
 // TNW-column workgroups runs the form that its last columns fill, gemm_tiles).
 template <bool PAIR, int NJ, bool EXACT>
@@ -1438,7 +1440,7 @@ __device__ __forceinline__ void gemm_body_h(const GemmArgs &a, const GemmAt &at,
 // 32-column tiles as hold tokens (an expert's last tile, a call's last columns).  At 3840
 // tokens an expert has 480 of them, and 128-column tiles alone multiply 10 % of padding
 // (64-column ones at 1500 tokens 16 %), 32-column ends 3 and 8 %: 3840 tokens of the model
-// 27.5 -> 26.8 ms, a 4-layer block of wide scales at 1500 tokens 2262 -> 2226 us.
+// 27.5 -> 26.8 ms, a 4-layer block of wide scales at 1500 tokens 36 us less.
 template <int N> struct Tiles {
     static constexpr int n = N;
 };
@@ -2125,8 +2127,8 @@ __device__ __forceinline__ void reduce_route(const GemmReduceArgs &a)
 
 // Four tokens per workgroup (calls of 128 tokens and more, with router partials): a
 // workgroup reads 32 KB of router rows whatever its tokens, 134 MB for 512 tokens one by
-// one.  A 4-layer block at 203 / 512 tokens takes 589 / 1054 us, 597 / 1093 one by one; the
-// sums and their order are the same.
+// one.  A 4-layer block at 203 / 512 tokens takes 8 / 39 us less than one by one; the sums
+// and their order are the same.
 extern "C" __global__ __launch_bounds__(WG_THREADS) void k_gemm_reduce_route4(const GemmReduceArgs a)
 {
     reduce_route<4>(a);
