@@ -887,11 +887,12 @@ __device__ __forceinline__ GemmAt gemm_at(const GemmArgs &a)
 // Grouped small calls: only the token tiles that the experts' lists fill are items (tiles
 // of ncol columns), counted here from the lists' lengths by every wave, so that the XCDs'
 // shares are equal whatever the routing; the launch has workgroups for the most tiles a
-// routing can need, and the others end here.  With every possible tile an item each XCD
-// had four experts: for 7 tokens, with about 19 experts in use, the busiest XCD had 1.7 -
-// 1.9 times the mean, and the gate/up pair took 53 us instead of 45 (203 tokens: 73 instead of
-// 60).  Large calls keep the experts whole: their lists differ by 5 % from XCD to XCD and
-// 3840 tokens of the model took 28.7 ms dealt out like this, 28.0 ms as they are.
+// routing can need, and the others end here.  With every possible tile an item each XCD had
+// four experts: for 7 tokens, with about 19 experts in use, the busiest XCD had 1.7 - 1.9
+// times the mean, and the gate/up pair took 8 us more (of 49 now with whole-range scales;
+// 203 tokens: 13 more, of 60 with narrow ones).  Large calls keep the experts whole: their
+// lists differ by 5 % from XCD to XCD and 3840 tokens of the model took 28.7 ms dealt out
+// like this, 28.0 ms as they are.
 __device__ __forceinline__ GemmAt gemm_at_group(const GemmArgs &a, uint32_t gx, uint32_t ncol)
 {
     const uint32_t lane = threadIdx.x & 63, c = lane < a.nz ? a.counts[lane] : 0u;
